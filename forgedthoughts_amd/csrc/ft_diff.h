@@ -55,6 +55,21 @@ struct DiffArgs {
   float lx, ly, lz;       // unit light direction
 };
 
+// Which product of a sum is fused is written out: left to the compiler it depends on the code
+// around (z or y of a length first), a last bit of a distance with it, and with that bit the
+// step at which a ray along a silhouette ends: of 60 fits of 32 spheres and 4 views at 320x320
+// one pixel in each of nine moved, the loss with it by up to 6e-4 and the gradient by 3.5e-3 of
+// its length.
+__device__ __forceinline__ float diff_dot(float3 a, float3 b) {
+  return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.x, b.x, a.y * b.y));
+}
+__device__ __forceinline__ float diff_len(float3 a) { return fsqrt(diff_dot(a, a)); }
+// sqrt(ux^2 + uy^2) and the value of op_union_round with r = max(|k|, 1e-6)
+__device__ __forceinline__ float diff_corner(float ux, float uy) { return fsqrt(__builtin_fmaf(ux, ux, uy * uy)); }
+__device__ __forceinline__ float diff_join(float a, float b, float r) {
+  return fmaxf(r, fminf(a, b)) - diff_corner(fmaxf(r - a, 0.0f), fmaxf(r - b, 0.0f));
+}
+
 // What a lane keeps of the cells while it evaluates the tree.
 struct DiffView {
   float ox, oy, oz, inv;
@@ -140,16 +155,14 @@ __device__ __forceinline__ float diff_eval(const DiffView& V, float3 p, DiffStar
         *st = top;
         st += 64;
       }
-      top = len(mk(p.x - cur.s.x, p.y - cur.s.y, p.z - cur.s.z)) - cur.s.w;
+      top = diff_len(mk(p.x - cur.s.x, p.y - cur.s.y, p.z - cur.s.z)) - cur.s.w;
     } else if (both) {
       st -= 64;
       a = *st;
     }
     if (join) {
       // a single operand x: op_union_round(x, infinity)
-      const float r = __uint_as_float(cur.w.y), other = both ? a : __builtin_huge_valf();
-      const float ux = fmaxf(r - other, 0.0f), uy = fmaxf(r - top, 0.0f);
-      top = fmaxf(r, fminf(other, top)) - fsqrt(ux * ux + uy * uy);
+      top = diff_join(both ? a : __builtin_huge_valf(), top, __uint_as_float(cur.w.y));
     }
     cur.w = cur.next;
     cur.next = after;
@@ -162,7 +175,7 @@ __device__ __forceinline__ float diff_eval(const DiffView& V, float3 p, DiffStar
 __device__ __forceinline__ void union_round_partials(float av, float bv, float r, float& da, float& db, float& dr) {
   const float ux = fmaxf(r - av, 0.0f), uy = fmaxf(r - bv, 0.0f);
   const float m = fminf(av, bv);
-  const float L = fsqrt(ux * ux + uy * uy);
+  const float L = diff_corner(ux, uy);
   da = (m > r && av <= bv) ? 1.0f : 0.0f;
   db = (m > r && !(av <= bv)) ? 1.0f : 0.0f;
   dr = m > r ? 0.0f : 1.0f;
@@ -263,7 +276,7 @@ __device__ __forceinline__ float diff_reverse(const DiffArgs& a, const DiffView&
         *st = top;
         st += 64;
       }
-      top = len(mk(p.x - cur.s.x, p.y - cur.s.y, p.z - cur.s.z)) - cur.s.w;
+      top = diff_len(mk(p.x - cur.s.x, p.y - cur.s.y, p.z - cur.s.z)) - cur.s.w;
     } else if (both) {
       st -= 64;
       x = *st;
@@ -271,8 +284,7 @@ __device__ __forceinline__ float diff_reverse(const DiffArgs& a, const DiffView&
     if (join) {
       const float r = __uint_as_float(cur.w.y), other = both ? x : __builtin_huge_valf();
       tr.put(k, other, top);
-      const float ux = fmaxf(r - other, 0.0f), uy = fmaxf(r - top, 0.0f);
-      top = fmaxf(r, fminf(other, top)) - fsqrt(ux * ux + uy * uy);
+      top = diff_join(other, top, r);
     }
     cur.w = cur.next;
     cur.next = after;
@@ -313,7 +325,7 @@ __device__ __forceinline__ float diff_reverse(const DiffArgs& a, const DiffView&
     if (prim) {
       const float4 s = global_load4(V.spheres, w.x & kDiffIndex);
       const float3 q = mk(p.x - s.x, p.y - s.y, p.z - s.z);
-      const float l = len(q);
+      const float l = diff_len(q);
       if (l > 0.0f) u = mul(q, 1.0f / l);
       grad = add(grad, mul(u, own));
       if (!both && st != V.stack) {  // the sphere began an operand of its own
@@ -384,7 +396,7 @@ __device__ __forceinline__ void diff_cells_body(const DiffArgs& a) {
     int wt, mark = 0;
     float vlo, vhi;
     if (d.x >= 0) {
-      const float f = len(mk(c.x - th[4 * d.x], c.y - th[4 * d.x + 1], c.z - th[4 * d.x + 2])) - th[4 * d.x + 3];
+      const float f = diff_len(mk(c.x - th[4 * d.x], c.y - th[4 * d.x + 1], c.z - th[4 * d.x + 2])) - th[4 * d.x + 3];
       wt = sp++ & (kDiffStack - 1);
       vlo = f - R;
       vhi = f + R;
@@ -510,9 +522,9 @@ __device__ __forceinline__ void diff_forward_body(DiffArgs a, float* __restrict_
             tans[sp++] = tan;
           }
           const float3 q = mk(m.pos.x - cur.s.x, m.pos.y - cur.s.y, m.pos.z - cur.s.z);
-          const float l = len(q);
+          const float l = diff_len(q);
           top = l - cur.s.w;
-          tan = l > 0.0f ? dot(mul(q, 1.0f / l), d) : 0.0f;
+          tan = l > 0.0f ? diff_dot(mul(q, 1.0f / l), d) : 0.0f;
         } else if (both) {
           st -= 64;
           av = *st;
@@ -522,8 +534,7 @@ __device__ __forceinline__ void diff_forward_body(DiffArgs a, float* __restrict_
           const float r = __uint_as_float(cur.w.y), other = both ? av : __builtin_huge_valf();
           float da, db, dr;
           union_round_partials(other, top, r, da, db, dr);
-          const float ux = fmaxf(r - other, 0.0f), uy = fmaxf(r - top, 0.0f);
-          top = fmaxf(r, fminf(other, top)) - fsqrt(ux * ux + uy * uy);
+          top = diff_join(other, top, r);
           tan = both ? da * at + db * tan : db * tan;
         }
         cur.w = cur.next;
@@ -544,9 +555,9 @@ __device__ __forceinline__ void diff_forward_body(DiffArgs a, float* __restrict_
         g[2] = k == 2 ? diff : g[2];
       }
       const float3 G = mk(g[0], g[1], g[2]);
-      const float gl = len(G);
+      const float gl = diff_len(G);
       const float3 n = gl > 1.0e-12f ? mul(G, 1.0f / gl) : mk(0.0f, 1.0f, 0.0f);
-      shade = fmaxf(dot(n, mk(a.lx, a.ly, a.lz)), 0.0f);
+      shade = fmaxf(diff_dot(n, mk(a.lx, a.ly, a.lz)), 0.0f);
     }
   }
   if (kCounted) diff_count(a, inside ? n_evals + (h ? 6 : 0) : 0, h ? 1 : 0, 0, flops);
@@ -616,11 +627,11 @@ __device__ __forceinline__ void diff_adjoint_body(DiffArgs a, const float* __res
         G = mk(k == 0 ? diff : G.x, k == 1 ? diff : G.y, k == 2 ? diff : G.z);
       }
     }
-    const float gl = len(G);
+    const float gl = diff_len(G);
     float3 v = mk(0.0f, 0.0f, 0.0f);
     if (gl > 1.0e-12f) {
       const float3 n = mul(G, 1.0f / gl);
-      const float nl = dot(n, l);
+      const float nl = diff_dot(n, l);
       if (nl > 0.0f) v = mul(sub(l, mul(n, nl)), gs / gl);
     }
     float c = 0.0f;
@@ -634,10 +645,10 @@ __device__ __forceinline__ void diff_adjoint_body(DiffArgs a, const float* __res
       diff_reverse<true>(a, V, tr, acc, start,
                          mk(xs.x + (axis == 0 ? off : 0.0f), xs.y + (axis == 1 ? off : 0.0f), xs.z + (axis == 2 ? off : 0.0f)),
                          seed, seed != 0.0f, g);
-      c += seed * dot(g, d);
+      c += seed * diff_dot(g, d);
     }
     diff_reverse<false>(a, V, tr, acc, start, xs, 0.0f, active, g);
-    const float gd = dot(g, d);
+    const float gd = diff_dot(g, d);
     const float s0 = (active && fabsf(gd) > 1.0e-6f) ? -(gt + c) / gd : 0.0f;
     diff_reverse<true>(a, V, tr, acc, start, xs, s0, s0 != 0.0f, g);
     if (kCounted) diff_count(a, active ? 6 : 0, active ? 1 : 0, active ? 7 : 0, flops);

@@ -230,3 +230,35 @@ def test_counted_kernels_match_and_count(small):
     per_eval = 10 * w.n_prims + 13 * (w.n_prims - 1)
     hits = int((t >= 0).sum())
     assert flops >= per_eval * (t.size + 16 * hits)
+
+
+# losses with every join of the tree evaluated at every point, lengths as fma(z, z, fma(x, x, y y))
+WHOLE_TREE_LOSS = {19: 38373.98785014648, 31: 42602.08975846099, 36: 28493.01545299478, 42: 23275.965396354408}
+
+
+@pytest.mark.parametrize("seed", list(WHOLE_TREE_LOSS))
+def test_loss_is_that_of_the_whole_tree(seed):
+    """Views with a ray along a silhouette that hits or misses on a last bit of a distance: rounded
+    another way, that pixel moves the loss by 3.6e-5 to 5.9e-4.  What the cells leave out cannot
+    show, so the distances are the whole tree's bit for bit.  The derivative of the Newton step may
+    round another way: a last bit of t* (2^-21 at most 8 away) in any of the N pixels moves
+    sum (t* - T)^2 by at most 2^-20 sqrt(N loss), 0.09 to 0.13 here: 4e-6 of the loss and less."""
+    rng = np.random.default_rng(seed)
+    target = np.concatenate([np.concatenate([rng.uniform(-2, 2, 3), rng.uniform(0.4, 0.9, 1)]) for _ in range(32)]
+                            + [rng.uniform(0.1, 0.4, 31)])
+    now = target + rng.normal(0, 0.05, target.size)
+    views = []
+    for _ in range(4):
+        z, phi = rng.uniform(-0.5, 0.9), rng.uniform(0, 2 * np.pi)
+        r = np.sqrt(1 - z * z)
+        views.append((0, (7 * r * np.cos(phi), 7 * z, 7 * r * np.sin(phi)), (0.0, 0.0, 0.0), 45.0))
+    opts = RenderOptions(width=320, height=320, max_steps=256, max_dist=30.0, epsilon=1e-5, step_scale=0.7,
+                         camera_z=6.0, fov_y_degrees=45.0)
+    print(f"[diff loss] seed {seed}, 32 prims, 4 views at 320^2", flush=True)
+    with DiffRenderer(32, views, opts) as dr:
+        dr.set_params(np.float32(target))
+        dr.set_target(*dr.forward())
+        dr.set_params(np.float32(now))
+        loss, _ = dr.loss_grad()
+    want = WHOLE_TREE_LOSS[seed]
+    assert abs(loss - want) <= 2.0 ** -20 * math.sqrt(4 * 320 * 320 * want), (loss, want)
