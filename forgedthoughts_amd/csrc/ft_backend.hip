@@ -755,9 +755,9 @@ int autotune_impl(ft_scene* s, uint32_t kind, const ft_render_options* o, const 
 struct CellScratch {
   DevBuf parents, words, marks, totals;
   int reset() {
-    int rc = ensure(totals, 2 * sizeof(unsigned));
+    int rc = ensure(totals, 2 * sizeof(CellTotal));
     if (rc) return rc;
-    FT_HIP(hipMemset(totals.ptr, 0, 2 * sizeof(unsigned)));
+    FT_HIP(hipMemset(totals.ptr, 0, 2 * sizeof(CellTotal)));
     FT_HIP(hipStreamSynchronize(nullptr));
     return FT_OK;
   }
@@ -801,8 +801,8 @@ void set_grid(DevScene& d, const fth::HostScene& h, int kind) {
 }
 
 // The counters of a count / write pair of launches: read and cleared in between.
-int read_totals(hipStream_t stream, DevBuf& totals, unsigned t[2]) {
-  const unsigned zero[2] = {0, 0};
+int read_totals(hipStream_t stream, DevBuf& totals, CellTotal t[2]) {
+  const CellTotal zero[2] = {0, 0};
   FT_HIP(hipGetLastError());
   FT_HIP(hipStreamSynchronize(stream));
   FT_HIP(hipMemcpy(t, totals.ptr, sizeof(zero), hipMemcpyDeviceToHost));
@@ -823,12 +823,12 @@ int build_leaf_lists(ft_scene* s, CellScratch& x) {
   const dim3 waves((unsigned)((n_parents + 63) / 64)), wave(64);
   const float4* prims = (const float4*)s->leaf_prims.ptr;
   const float4* boxes = (const float4*)s->leaf_boxes.ptr;
-  unsigned t[2];
+  CellTotal t[2];
   if ((rc = x.reset()) || (rc = ensure(x.parents, (size_t)n_parents * sizeof(int4)))) return rc;
-  unsigned* totals = (unsigned*)x.totals.ptr;
+  CellTotal* totals = (CellTotal*)x.totals.ptr;
   hipLaunchKernelGGL(ft_k_leaf_parents_count, waves, wave, 0, s->stream, g, prims, boxes, np, n, (int4*)x.parents.ptr, totals);
   if ((rc = read_totals(s->stream, x.totals, t))) return rc;
-  if (t[1] > 0x7fffu || t[0] > (1u << 31) / 64) return FT_OK;
+  if (t[1] > kLongestList || t[0] > (1u << 31) / 64) return FT_OK;  // 64 children of at most as many: below 2^31
   if ((rc = ensure(x.words, ((size_t)t[0] + 4) * sizeof(unsigned)))) return rc;
   hipLaunchKernelGGL(ft_k_leaf_parents_write, waves, wave, 0, s->stream, g, prims, boxes, np, n, (int4*)x.parents.ptr,
                      (unsigned*)x.words.ptr, totals);
@@ -837,7 +837,7 @@ int build_leaf_lists(ft_scene* s, CellScratch& x) {
   hipLaunchKernelGGL(ft_k_leaf_children_count, dim3(n_parents), wave, 0, s->stream, g, prims, boxes, np, n,
                      (const int4*)x.parents.ptr, (const unsigned*)x.words.ptr, (int4*)s->cell_lists.ptr, totals);
   if ((rc = read_totals(s->stream, x.totals, t))) return rc;
-  if ((double)t[0] > 64.0 * (double)n_cells || t[1] > 0x7fffu) return FT_OK;
+  if ((double)t[0] > 64.0 * (double)n_cells || t[1] > kLongestList) return FT_OK;
   if ((rc = ensure(s->cell_items, ((size_t)t[0] + 4) * sizeof(unsigned)))) return rc;
   hipLaunchKernelGGL(ft_k_leaf_children_write, dim3(n_parents), wave, 0, s->stream, g, prims, boxes, np, n,
                      (const int4*)x.parents.ptr, (const unsigned*)x.words.ptr, (int4*)s->cell_lists.ptr,
@@ -948,11 +948,11 @@ int build_cell_programs(ft_scene* s, CellScratch& x) {
   const dim3 waves((unsigned)((n_parents + 63) / 64)), wave(64);
   const DOp* ops = (const DOp*)s->ops.ptr;
   int rc;
-  unsigned t[2];
+  CellTotal t[2];
   if ((rc = x.reset()) || (rc = ensure(x.parents, (size_t)n_parents * sizeof(int2))) ||
       (rc = ensure(x.marks, (size_t)((n_prog + 7) / 8) * n_parents * sizeof(unsigned))))
     return rc;
-  unsigned* totals = (unsigned*)x.totals.ptr;
+  CellTotal* totals = (CellTotal*)x.totals.ptr;
   int2* parents = (int2*)x.parents.ptr;
   hipLaunchKernelGGL(ft_k_cell_parents_count, waves, wave, 0, s->stream, g, ops, n_prog, (unsigned*)x.marks.ptr, parents, totals);
   if ((rc = read_totals(s->stream, x.totals, t))) return rc;
@@ -970,7 +970,7 @@ int build_cell_programs(ft_scene* s, CellScratch& x) {
   hipLaunchKernelGGL(ft_k_cell_children_count, dim3(n_parents), wave, 0, s->stream, g, ops, (const int2*)parents, from,
                      (unsigned*)x.marks.ptr, (int4*)s->cell_progs.ptr, (int2*)s->cell_shades.ptr, totals);
   if ((rc = read_totals(s->stream, x.totals, t))) return rc;
-  if ((double)t[1] > 0.25 * (double)n_prog * (double)n_cells) return FT_OK;
+  if ((double)t[1] > 0.25 * (double)n_prog * (double)n_cells || t[0] + 4ull * n_prog > (1u << 31)) return FT_OK;
   // the whole program in front, then the cells', and room to read ahead at the end
   std::vector<unsigned> whole;
   for (int k = 0; k < n_prog; ++k) {
@@ -991,7 +991,7 @@ int build_cell_programs(ft_scene* s, CellScratch& x) {
     whole.push_back(is_prim(kind) ? prim_word(h.ops[k], k) : join_word(kind, kOneBoth) | (unsigned)k);
   }
   if (whole.size() & 1) whole.push_back(0u);
-  const unsigned cursor = (unsigned)whole.size();
+  const CellTotal cursor = whole.size();
   const int4 all = make_int4((int)whole[0], (int)whole[1], 2, n_whole);
   const int2 all_shades = make_int2(2 * n_whole, n_prog);
   if ((rc = upload(s->cell_ops, h.cell_ops)) || (rc = upload(s->cell_ext, h.cell_ext)) ||

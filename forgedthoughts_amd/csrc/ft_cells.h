@@ -475,8 +475,15 @@ __device__ __forceinline__ float3 child_centre(const CellGrid& g, int i, int lan
   return cell_centre(g, g.cell, x, y, z);
 }
 
+// The counters of a build, [0] words and [1] what the host decides by beside them.  They hold
+// more than 32 bits: whether a build's words fit is decided from their whole count.
+typedef unsigned long long CellTotal;
+// A leaf list has at most this many entries of a kind, since its two counts share a word; scenes
+// with longer ones keep the BVH walk.
+constexpr int kLongestList = 0x7fff;
+
 // Room for `n` words from a counter, one atomic per wave.
-__device__ __forceinline__ unsigned take_room(unsigned* cursor, unsigned n) {
+__device__ __forceinline__ unsigned take_room(CellTotal* cursor, unsigned n) {
   unsigned incl = n;
   const int lane = (int)(threadIdx.x & 63u);
 #pragma unroll
@@ -485,14 +492,14 @@ __device__ __forceinline__ unsigned take_room(unsigned* cursor, unsigned n) {
     if (lane >= m) incl += v;
   }
   unsigned base = 0u;
-  if (lane == 63) base = atomicAdd(cursor, incl);
+  if (lane == 63) base = (unsigned)atomicAdd(cursor, (CellTotal)incl);
   return __shfl(base, 63, 64) + incl - n;
 }
 
 // The leaf lists of one cell with centre c and radius R.  The candidates are `source` (null: all
 // sorted leaves, [0, n_prims) primitives, [n_prims, n) known by their bounds only) for the
 // distances and `source_box` for the bounds, read in step by the whole wave.  kWrite = false
-// counts; kWrite = true writes to the room taken in `r`.
+// counts, the longer of the first two lists in `longest`; kWrite = true writes to the room taken in `r`.
 struct LeafSource {
   const unsigned* items;  // null: leaf k is k
   int n_prims, n_others, n_boxes;
@@ -501,7 +508,7 @@ struct LeafSource {
 template <bool kWrite>
 __device__ __forceinline__ void leaf_lists_cell(const LeafSource& s, const float4* __restrict__ prims,
                                                 const float4* __restrict__ boxes, unsigned none, float3 c, float R, bool mine,
-                                                int4& r, unsigned* __restrict__ items) {
+                                                int4& r, int& longest, unsigned* __restrict__ items) {
   const auto P = uniform_ptr(prims);
   const auto X = uniform_ptr(boxes);
   const auto I = uniform_ptr(s.items);
@@ -545,18 +552,21 @@ __device__ __forceinline__ void leaf_lists_cell(const LeafSource& s, const float
     for (; no < want_o; ++no) items[r.x + pad + no] = none;
     for (; nb < want_b; ++nb) items[r.z + nb] = none;
   }
-  if (!kWrite) r = make_int4(0, np | (no << 16), 0, nb);
+  if (!kWrite) {
+    longest = max(np, no);
+    r = make_int4(0, min(np, kLongestList) | (min(no, kLongestList) << 16), 0, nb);
+  }
 }
 
 // Parents (kChild = false: 64 of them per wave, from all leaves) or their children (a wave per
 // parent, from its lists `from` / `from_items`).  Counting adds the words needed to totals[0]
-// and the longest list to totals[1]; writing takes room at totals[0].
+// and the longest list of either kind to totals[1]; writing takes room at totals[0].
 template <bool kWrite, bool kChild>
 __device__ __forceinline__ void leaf_lists_body(CellGrid g, const float4* __restrict__ prims,
                                                 const float4* __restrict__ boxes, int n_prims, int n,
                                                 const int4* __restrict__ from, const unsigned* __restrict__ from_items,
                                                 int4* __restrict__ lists, unsigned* __restrict__ items,
-                                                unsigned* __restrict__ totals) {
+                                                CellTotal* __restrict__ totals) {
   const int lane = (int)threadIdx.x, n_parents = g.px * g.py * g.pz;
   LeafSource s{nullptr, n_prims, n - n_prims, n, 0u, (unsigned)n_prims, 0u};
   int index;
@@ -583,11 +593,12 @@ __device__ __forceinline__ void leaf_lists_body(CellGrid g, const float4* __rest
     r.x = (int)take_room(&totals[0], mine ? words(r) : 0u);
     r.z = r.x + (((r.y & 0xffff) + 1) & ~1) + (r.y >> 16);
   }
-  leaf_lists_cell<kWrite>(s, prims, boxes, (unsigned)n, c, R, mine, r, items);
+  int longest = 0;
+  leaf_lists_cell<kWrite>(s, prims, boxes, (unsigned)n, c, R, mine, r, longest, items);
   if (mine) lists[index] = r;
   if (!kWrite && mine) {
-    atomicAdd(&totals[0], words(r));
-    atomicMax(&totals[1], (unsigned)max(r.y & 0xffff, r.y >> 16));
+    atomicAdd(&totals[0], (CellTotal)words(r));
+    atomicMax(&totals[1], (CellTotal)longest);
   }
 }
 
@@ -761,7 +772,7 @@ __device__ __forceinline__ void cell_program(const DOp* __restrict__ ops_, const
 template <bool kWrite>
 __device__ __forceinline__ void cell_parents_body(CellGrid g, const DOp* __restrict__ ops, int n_prog,
                                                   unsigned* __restrict__ marks, int2* __restrict__ parents,
-                                                  unsigned* __restrict__ words, unsigned* __restrict__ totals) {
+                                                  unsigned* __restrict__ words, CellTotal* __restrict__ totals) {
   const int n_parents = g.px * g.py * g.pz;
   const int i = (int)blockIdx.x * 64 + (int)threadIdx.x;
   const bool mine = i < n_parents;
@@ -772,14 +783,14 @@ __device__ __forceinline__ void cell_parents_body(CellGrid g, const DOp* __restr
   cell_program<kWrite, true>(ops, nullptr, n_prog, parent_centre(g, m), cell_radius(g, g.cell * kCellChildren),
                              0.25f * g.margin, mine, marks + m, n_parents, r, sh, words);
   if (mine) parents[m] = sh;
-  if (!kWrite && mine) atomicAdd(&totals[0], (unsigned)(sh.y + 7) & ~7u);
+  if (!kWrite && mine) atomicAdd(&totals[0], (CellTotal)((unsigned)(sh.y + 7) & ~7u));
 }
 // Children (a wave per parent).  totals[0]: words, [1]: distance words alone.
 template <bool kWrite>
 __device__ __forceinline__ void cell_children_body(CellGrid g, const DOp* __restrict__ ops, const int2* __restrict__ parents,
                                                    const unsigned* __restrict__ parent_words, unsigned* __restrict__ marks,
                                                    int4* __restrict__ progs, int2* __restrict__ shades,
-                                                   unsigned* __restrict__ words, unsigned* __restrict__ totals) {
+                                                   unsigned* __restrict__ words, CellTotal* __restrict__ totals) {
   const int p = __builtin_amdgcn_readfirstlane((int)blockIdx.x);
   int index;
   const float3 c = child_centre(g, p, (int)threadIdx.x, index);
@@ -797,8 +808,8 @@ __device__ __forceinline__ void cell_children_body(CellGrid g, const DOp* __rest
   progs[index] = r;
   shades[index] = sh;
   if (!kWrite) {
-    atomicAdd(&totals[0], (unsigned)(2 * (r.w - 1) + ((sh.y + 1) & ~1)));
-    atomicAdd(&totals[1], (unsigned)r.w);
+    atomicAdd(&totals[0], (CellTotal)(2 * (r.w - 1) + ((sh.y + 1) & ~1)));
+    atomicAdd(&totals[1], (CellTotal)r.w);
   }
 }
 

@@ -563,38 +563,38 @@ FT_KERNEL FT_MARCH_OCCUPANCY void ft_k_atlas_bricks(int slot, ftd::AtlasGrid g, 
 }
 #define FT_CELL_KERNEL extern "C" __global__ __launch_bounds__(64)
 FT_CELL_KERNEL void ft_k_leaf_parents_count(ftd::CellGrid g, const float4* prims, const float4* boxes, int n_prims, int n,
-                                            int4* lists, unsigned* totals) {
+                                            int4* lists, ftd::CellTotal* totals) {
   ftd::leaf_lists_body<false, false>(g, prims, boxes, n_prims, n, nullptr, nullptr, lists, nullptr, totals);
 }
 FT_CELL_KERNEL void ft_k_leaf_parents_write(ftd::CellGrid g, const float4* prims, const float4* boxes, int n_prims, int n,
-                                            int4* lists, unsigned* items, unsigned* totals) {
+                                            int4* lists, unsigned* items, ftd::CellTotal* totals) {
   ftd::leaf_lists_body<true, false>(g, prims, boxes, n_prims, n, nullptr, nullptr, lists, items, totals);
 }
 FT_CELL_KERNEL void ft_k_leaf_children_count(ftd::CellGrid g, const float4* prims, const float4* boxes, int n_prims, int n,
-                                             const int4* from, const unsigned* from_items, int4* lists, unsigned* totals) {
+                                             const int4* from, const unsigned* from_items, int4* lists, ftd::CellTotal* totals) {
   ftd::leaf_lists_body<false, true>(g, prims, boxes, n_prims, n, from, from_items, lists, nullptr, totals);
 }
 FT_CELL_KERNEL void ft_k_leaf_children_write(ftd::CellGrid g, const float4* prims, const float4* boxes, int n_prims, int n,
                                              const int4* from, const unsigned* from_items, int4* lists, unsigned* items,
-                                             unsigned* totals) {
+                                             ftd::CellTotal* totals) {
   ftd::leaf_lists_body<true, true>(g, prims, boxes, n_prims, n, from, from_items, lists, items, totals);
 }
 FT_CELL_KERNEL void ft_k_cell_parents_count(ftd::CellGrid g, const ftd::DOp* ops, int n_prog, unsigned* marks, int2* parents,
-                                            unsigned* totals) {
+                                            ftd::CellTotal* totals) {
   ftd::cell_parents_body<false>(g, ops, n_prog, marks, parents, nullptr, totals);
 }
 FT_CELL_KERNEL void ft_k_cell_parents_write(ftd::CellGrid g, const ftd::DOp* ops, int n_prog, unsigned* marks, int2* parents,
-                                            unsigned* words, unsigned* totals) {
+                                            unsigned* words, ftd::CellTotal* totals) {
   ftd::cell_parents_body<true>(g, ops, n_prog, marks, parents, words, totals);
 }
 FT_CELL_KERNEL void ft_k_cell_children_count(ftd::CellGrid g, const ftd::DOp* ops, const int2* parents,
                                              const unsigned* parent_words, unsigned* marks, int4* progs, int2* shades,
-                                             unsigned* totals) {
+                                             ftd::CellTotal* totals) {
   ftd::cell_children_body<false>(g, ops, parents, parent_words, marks, progs, shades, nullptr, totals);
 }
 FT_CELL_KERNEL void ft_k_cell_children_write(ftd::CellGrid g, const ftd::DOp* ops, const int2* parents,
                                              const unsigned* parent_words, unsigned* marks, int4* progs, int2* shades,
-                                             unsigned* words, unsigned* totals) {
+                                             unsigned* words, ftd::CellTotal* totals) {
   ftd::cell_children_body<true>(g, ops, parents, parent_words, marks, progs, shades, words, totals);
 }
 FT_KERNEL void ft_k_clear_flag(int* flag) { ftd::clear_flag_body(flag); }

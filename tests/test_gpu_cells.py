@@ -17,7 +17,7 @@ from forgedthoughts_amd.options import AccelMode, RaySettings, RenderOptions
 from forgedthoughts_amd.render import GpuScene
 from oracle import ftref
 
-from helpers import compile_src
+from helpers import compile_src, with_camera
 
 pytestmark = pytest.mark.gpu
 
@@ -76,6 +76,51 @@ def parts_scene(n, seed, odd, eye, extent=2.5):
             text += primitive(rng, f"p{k}", extent, k >= odd, f"m{k}")
         names.append(f"p{k}")
     return text + f"let scene = {tree(names, lambda a, b: f'({a} + {b})')};\n"
+
+
+def spheres_scene(centres, radii):
+    """Separate spheres in a balanced tree of hard unions, without going through the source text."""
+    s = compile_src(LIGHTS + "let m = Lambert { color: vec3(0.8, 0.5, 0.3) };\nvar a = Sphere { radius: 1.0, material: m };\n"
+                    "var b = Sphere { radius: 1.0, material: m };\nlet scene = (a + b);\n")
+    leaf, union = s.nodes[s.nodes["lhs"] < 0][0], s.nodes[s.root]
+    nodes = np.empty(2 * len(centres) - 1, dtype=s.nodes.dtype)
+    n = 0
+
+    def build(lo, hi):
+        nonlocal n
+        if hi - lo == 1:
+            rec = leaf.copy()
+            rec["center"], rec["param"][0] = centres[lo], radii[lo]
+        else:
+            mid = (lo + hi) // 2
+            rec = union.copy()
+            rec["lhs"], rec["rhs"] = build(lo, mid), build(mid, hi)
+        nodes[n] = rec
+        n += 1
+        return n - 1
+    s.root, s.nodes, s.leaf_count, s._ir = build(0, len(centres)), nodes, len(centres), None
+    return s
+
+
+@pytest.mark.parametrize("n", [32700, 66000])
+def test_lists_of_more_leaves_than_their_counts_hold(n):
+    """A clump far smaller than a cell among scattered spheres: every cell near it keeps the whole clump.
+    The two counts of a list share a word, 15 bits each: 66 000 (464 in 16 bits, and a carry into the
+    other count) have to leave the lists unused, 32 700 are the most that one may hold."""
+    rng = np.random.default_rng(1)
+    clump = rng.uniform(-0.02, 0.02, (n, 3)) + rng.uniform(-25, 25, 3)
+    far = rng.uniform(-50, 50, (5000, 3))
+    scene = spheres_scene(np.concatenate([clump, far]), np.concatenate([np.full(n, 0.002), rng.uniform(0.15, 0.5, 5000)]))
+    at = clump.mean(0)
+    scene = with_camera(scene, at + (0.02, 0.03, -0.08), at, 45.0)
+    opts = RenderOptions(width=24, height=24, **{**OPTS, "epsilon": 1.0e-4})
+    print(f"[leaf lists] a clump of {n}", flush=True)
+    with GpuScene(scene, AccelMode.Bvh) as gs:
+        _, t = gs.render_depth(opts, 1)
+    _, want = ftref.render_depth(scene, AccelMode.Bvh, opts, 1)
+    hit = want >= 0
+    assert hit.sum() > 200 and np.array_equal(t >= 0, hit)
+    assert np.abs(t - want)[hit].max() <= 1.0e-4
 
 
 JOINS = ["union_round", "union_chamfer", "union_stairs", "union_soft", "diff_round", "diff_chamfer", "diff_stairs",
