@@ -121,6 +121,7 @@ struct ft_scene {
   int* last_overflow = nullptr;  // overflow flag of the last Whitted render, read by finish()
   // scene specialisation
   fth::EmitPlan plan;
+  bool straight = false;  // emitted, and a scene whose distance straight-line code can be (cells may answer it instead)
   std::string source;                              // emitted translation unit (empty: interpreter)
   // runtime-compiled code objects, one per (kernel, counted, occupancy, unroll), built on
   // first use: the scene-specialised kernels, the *_counted variants (FLOP counting on) and
@@ -1106,7 +1107,7 @@ static int create_scene(const ft_scene_ir* ir, uint32_t accel_mode, bool batch_m
     const bool always = m == "1" || m == "always", never = m == "0" || m == "never";
     s->plan = fth::plan_emission(h, ir);
     bool emit = !batch_member && (always ? s->plan.any() : (!never && s->plan.any() && fth::emission_pays(h, ir, s->plan)));
-    const bool straight = emit && s->plan.scene;  // the distance could run as straight-line code
+    const bool straight = s->straight = emit && s->plan.scene;
     if (!h.leaf_prims.empty()) rc = build_leaf_lists(s, scratch);
     else if (h.cell_programs && (!straight || (!always && (int)h.prog.size() >= kCellDepthNodes)))
       rc = build_cell_programs(s, scratch);
@@ -1252,7 +1253,7 @@ int ft_scene_stats(ft_scene* s, ft_render_stats* out) {
   *out = s->stats;
   out->flags = 0;
   if (!s->source.empty()) {
-    if (s->plan.scene) out->flags |= FT_STATS_EMITTED_SCENE;
+    if (s->straight) out->flags |= FT_STATS_EMITTED_SCENE;
     if (s->plan.functions) out->flags |= FT_STATS_EMITTED_FUNCTIONS;
   }
   out->compile_ms = s->compile_ms;

@@ -318,7 +318,8 @@ class GpuBatch:
 
 
 def emit_scene_source(scene: CompiledScene, accel: AccelMode = AccelMode.Bvh) -> str:
-    """The scene-specialised HIP translation unit the backend would compile for `scene`."""
+    """The scene-specialised HIP translation unit of `scene` (FT_EMIT=1; by itself the backend
+    leaves the distance and the sweep out where the scene's cells answer them)."""
     ir = scene.ir()
     n = C.c_uint64(0)
     _check(library().ft_emit_scene_source(C.addressof(ir), int(accel), None, 0, C.byref(n)))

@@ -455,7 +455,10 @@ typedef struct ft_render_stats {
   uint64_t atlas_bricks;  /* bricks in the atlas */
   uint32_t ray_stack;     /* ray-stack entries of the last Whitted kernel (ft_k_whitted_N), 0: none yet */
 } ft_render_stats;
-#define FT_STATS_EMITTED_SCENE 1u     /* scene distance runs as specialised straight-line code */
+/* Both say that Whitted kernels of the scene are built at run time, before their first use
+ * (ft_render_whitted_device_noalloc refuses until then). */
+#define FT_STATS_EMITTED_SCENE 1u     /* distance and shading are specialised to the scene: straight-line
+                                       * code, or in larger trees spatial cells and code beside them */
 #define FT_STATS_EMITTED_FUNCTIONS 2u /* Forge functions run as specialised code */
 int ft_scene_stats(ft_scene* scene, ft_render_stats* out);
 
@@ -544,7 +547,8 @@ int ft_diff_set_flop_counting(ft_diff* diff, int enable);
 
 /* Scene specialisation diagnostics (no GPU needed).  ft_emit_scene_source writes the
  * translation unit the emitter produces for `ir` under `accel_mode` (always emitted, the
- * FT_EMIT policy aside) into buf (cap bytes, NUL-terminated, *len_out = full length);
+ * FT_EMIT policy aside; where spatial cells answer the distance of a scene, the backend
+ * compiles the unit without it) into buf (cap bytes, NUL-terminated, *len_out = full length);
  * ft_emit_compile additionally compiles it with hiprtc for one kernel (0 depth, 1/2/3
  * Whitted with a 16/48/128-entry ray stack) and reports the compile time.  No counterpart
  * in the reference: its Cranelift JIT (crates/forgedthoughts/src/jit.rs) has no such hook;

@@ -248,7 +248,7 @@ def test_noalloc_with_cells_needs_a_built_kernel():
     rgb = torch.zeros(64 * 32 * 3, dtype=torch.uint8, device="cuda")
     o, rs = w.options.to_c(), w.settings.to_c()
     with GpuScene(scene, w.accel) as gs:
-        assert gs.stats().flags == abi.STATS_EMITTED_FUNCTIONS
+        assert gs.stats().flags == abi.STATS_EMITTED_SCENE | abi.STATS_EMITTED_FUNCTIONS
         gs.render_depth_device(w.options, 1, rgb.data_ptr())
         gs.synchronize()
         assert gs.stats().compile_ms == 0.0
@@ -264,6 +264,20 @@ def test_noalloc_with_cells_needs_a_built_kernel():
         assert call() == 0
         gs.synchronize()
         assert torch.equal(rgb, ref)
+
+
+def test_stats_say_when_kernels_are_built():
+    """A tree with cells, no function, and an intersection of unlike materials: of its kernels only
+    the shading sweep is compiled, and the flags have to say that one is."""
+    from forgedthoughts_amd import abi
+    text = tree_scene(60, 21, (1.0, 2.0, -6.5), ["union_round", "and"], ("Lambert", "Metal"), plain=True)
+    opts = RenderOptions(width=32, height=24, **OPTS)
+    with GpuScene(compile_src(text), AccelMode.Bvh) as gs:
+        gs.render_depth(opts, 1)
+        assert gs.stats().compile_ms == 0.0
+        assert gs.stats().flags == abi.STATS_EMITTED_SCENE
+        gs.render_whitted(opts, RaySettings(1, 64, 1))
+        assert gs.stats().compile_ms > 0.0
 
 
 # (text of the scene after the camera and lights, eye): one primitive; every primitive kind, rotated
