@@ -113,10 +113,11 @@ class RenderStatsC(C.Structure):
     _fields_ = [("primary_rays", C.c_uint64), ("kernel_launches", C.c_uint64),
                 ("last_kernel_ms", C.c_float), ("flags", C.c_uint32), ("sdf_flops", C.c_uint64),
                 ("compile_ms", C.c_double), ("atlas_samples", C.c_uint64), ("atlas_bytes", C.c_uint64),
-                ("atlas_bricks", C.c_uint64), ("ray_stack", C.c_uint32)]
+                ("atlas_bricks", C.c_uint64), ("ray_stack", C.c_uint32), ("cells", C.c_uint32)]
 
 
 STATS_EMITTED_SCENE, STATS_EMITTED_FUNCTIONS = 1, 2
+CELLS_NONE, CELLS_LISTS, CELLS_PROGRAMS, CELLS_TINY = range(4)
 
 
 class View(C.Structure):

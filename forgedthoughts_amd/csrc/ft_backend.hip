@@ -1257,6 +1257,7 @@ int ft_scene_stats(ft_scene* s, ft_render_stats* out) {
     if (s->plan.functions) out->flags |= FT_STATS_EMITTED_FUNCTIONS;
   }
   out->compile_ms = s->compile_ms;
+  out->cells = (uint32_t)s->dev.cells;
   return FT_OK;
 }
 

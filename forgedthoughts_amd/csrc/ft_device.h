@@ -79,7 +79,7 @@ struct DevScene {
   int n_tiny;
   int cell_sweep;                        // the shading sweep runs the cells' shading words
 };
-constexpr int kCellNone = 0, kCellLists = 1, kCellPrograms = 2, kCellTiny = 3;
+constexpr int kCellNone = FT_CELLS_NONE, kCellLists = FT_CELLS_LISTS, kCellPrograms = FT_CELLS_PROGRAMS, kCellTiny = FT_CELLS_TINY;
 
 // Scene descriptors live in constant memory, one slot per scene handle.  Device functions
 // receive the slot index and re-read it with readfirstlane, so every scene field is a

@@ -454,7 +454,13 @@ typedef struct ft_render_stats {
   uint64_t atlas_bytes;   /* device bytes of the scene's distance atlas (0: none) */
   uint64_t atlas_bricks;  /* bricks in the atlas */
   uint32_t ray_stack;     /* ray-stack entries of the last Whitted kernel (ft_k_whitted_N), 0: none yet */
+  uint32_t cells;         /* FT_CELLS_*: what the scene's distance comes from where no straight-line code
+                           * gives it (ft_scene_stats; 0 elsewhere) */
 } ft_render_stats;
+#define FT_CELLS_NONE 0u     /* the node program or the BVH */
+#define FT_CELLS_LISTS 1u    /* the leaves of the point's cell */
+#define FT_CELLS_PROGRAMS 2u /* the nodes of the point's cell */
+#define FT_CELLS_TINY 3u     /* a few words held in registers */
 /* Both say that Whitted kernels of the scene are built at run time, before their first use
  * (ft_render_whitted_device_noalloc refuses until then). */
 #define FT_STATS_EMITTED_SCENE 1u     /* distance and shading are specialised to the scene: straight-line
