@@ -751,10 +751,26 @@ int autotune_impl(ft_scene* s, uint32_t kind, const ft_render_options* o, const 
 
 }  // namespace
 
+// The device memory that the cells of one scene may take, of each kind of buffer (FT_CELL_MB, read
+// when a scene is created; 0: no cells and no tiny words).  Trees of up to 2048 blended parts, of which
+// a cell keeps a few, take 23 to 120 MB, one of 400 parts on top of each other 319: a gigabyte is
+// reached where much of a large tree remains in most cells, which then gain little.
+static size_t cell_memory() {
+  const char* env = std::getenv("FT_CELL_MB");
+  char* end = nullptr;
+  const unsigned long long mb = env ? std::strtoull(env, &end, 10) : 1024ull;
+  return (size_t)(env && (end == env || *end) ? 1024ull : std::min(mb, 1ull << 20)) << 20;
+}
+
 // Device memory used while a scene's cells are built: the parent cells and their words, the
 // marks, two counters.  A batch keeps one for all its scenes; freed before the call returns.
 struct CellScratch {
   DevBuf parents, words, marks, totals;
+  const size_t limit = cell_memory();
+  // `bytes` in b, FT_ERR_OUT_OF_MEMORY where that is above the limit as where there are none left
+  int room(DevBuf& b, size_t bytes) const {
+    return bytes > limit ? fail(FT_ERR_OUT_OF_MEMORY, "cells larger than FT_CELL_MB") : ensure(b, bytes);
+  }
   int reset() {
     int rc = ensure(totals, 2 * sizeof(CellTotal));
     if (rc) return rc;
@@ -762,10 +778,13 @@ struct CellScratch {
     FT_HIP(hipStreamSynchronize(nullptr));
     return FT_OK;
   }
-  ~CellScratch() {
-    for (DevBuf* b : {&parents, &words, &marks, &totals})
+  void drop() {
+    for (DevBuf* b : {&parents, &words, &marks, &totals}) {
       if (b->ptr) (void)hipFree(b->ptr);
+      *b = DevBuf();
+    }
   }
+  ~CellScratch() { drop(); }
 };
 
 static int create_scene(const ft_scene_ir* ir, uint32_t accel_mode, bool batch_member, CellScratch& scratch, ft_scene** out);
@@ -825,21 +844,21 @@ int build_leaf_lists(ft_scene* s, CellScratch& x) {
   const float4* prims = (const float4*)s->leaf_prims.ptr;
   const float4* boxes = (const float4*)s->leaf_boxes.ptr;
   CellTotal t[2];
-  if ((rc = x.reset()) || (rc = ensure(x.parents, (size_t)n_parents * sizeof(int4)))) return rc;
+  if ((rc = x.reset()) || (rc = x.room(x.parents, (size_t)n_parents * sizeof(int4)))) return rc;
   CellTotal* totals = (CellTotal*)x.totals.ptr;
   hipLaunchKernelGGL(ft_k_leaf_parents_count, waves, wave, 0, s->stream, g, prims, boxes, np, n, (int4*)x.parents.ptr, totals);
   if ((rc = read_totals(s->stream, x.totals, t))) return rc;
   if (t[1] > kLongestList || t[0] > (1u << 31) / 64) return FT_OK;  // 64 children of at most as many: below 2^31
-  if ((rc = ensure(x.words, ((size_t)t[0] + 4) * sizeof(unsigned)))) return rc;
+  if ((rc = x.room(x.words, ((size_t)t[0] + 4) * sizeof(unsigned)))) return rc;
   hipLaunchKernelGGL(ft_k_leaf_parents_write, waves, wave, 0, s->stream, g, prims, boxes, np, n, (int4*)x.parents.ptr,
                      (unsigned*)x.words.ptr, totals);
   if ((rc = read_totals(s->stream, x.totals, t))) return rc;
-  if ((rc = ensure(s->cell_lists, n_cells * sizeof(int4)))) return rc;
+  if ((rc = x.room(s->cell_lists, n_cells * sizeof(int4)))) return rc;
   hipLaunchKernelGGL(ft_k_leaf_children_count, dim3(n_parents), wave, 0, s->stream, g, prims, boxes, np, n,
                      (const int4*)x.parents.ptr, (const unsigned*)x.words.ptr, (int4*)s->cell_lists.ptr, totals);
   if ((rc = read_totals(s->stream, x.totals, t))) return rc;
   if ((double)t[0] > 64.0 * (double)n_cells || t[1] > kLongestList) return FT_OK;
-  if ((rc = ensure(s->cell_items, ((size_t)t[0] + 4) * sizeof(unsigned)))) return rc;
+  if ((rc = x.room(s->cell_items, ((size_t)t[0] + 4) * sizeof(unsigned)))) return rc;
   hipLaunchKernelGGL(ft_k_leaf_children_write, dim3(n_parents), wave, 0, s->stream, g, prims, boxes, np, n,
                      (const int4*)x.parents.ptr, (const unsigned*)x.words.ptr, (int4*)s->cell_lists.ptr,
                      (unsigned*)s->cell_items.ptr, totals);
@@ -858,7 +877,7 @@ int build_leaf_lists(ft_scene* s, CellScratch& x) {
 // samples, ms): 1 part 0.16 / 0.20 and 1.44 / 1.59, 4 parts 0.31 / 0.46 and 1.76 / 2.17,
 // 7 parts 0.38 / 0.44 and 1.96 / 2.19, a blend of 4 0.33 / 0.57 and 1.79 / 2.38, of 7
 // 0.61 / 0.66 and 2.63 / 2.78: beyond kTinyWords words the advantage is gone.
-int build_tiny(ft_scene* s) {
+int build_tiny(ft_scene* s, CellScratch&) {
   const fth::HostScene& h = s->host;
   const int n_prog = (int)h.prog.size(), n_leaves = (int)h.leaves.size();
   const bool naive = h.accel == FT_ACCEL_NAIVE;
@@ -950,8 +969,8 @@ int build_cell_programs(ft_scene* s, CellScratch& x) {
   const DOp* ops = (const DOp*)s->ops.ptr;
   int rc;
   CellTotal t[2];
-  if ((rc = x.reset()) || (rc = ensure(x.parents, (size_t)n_parents * sizeof(int2))) ||
-      (rc = ensure(x.marks, (size_t)((n_prog + 7) / 8) * n_parents * sizeof(unsigned))))
+  if ((rc = x.reset()) || (rc = x.room(x.parents, (size_t)n_parents * sizeof(int2))) ||
+      (rc = x.room(x.marks, (size_t)((n_prog + 7) / 8) * n_parents * sizeof(unsigned))))
     return rc;
   CellTotal* totals = (CellTotal*)x.totals.ptr;
   int2* parents = (int2*)x.parents.ptr;
@@ -959,13 +978,13 @@ int build_cell_programs(ft_scene* s, CellScratch& x) {
   if ((rc = read_totals(s->stream, x.totals, t))) return rc;
   const size_t n_from = t[0];
   if (n_from > (1ull << 31) / (64 * 3)) return FT_OK;  // 64 children of at most three words a node: below 2^31
-  if ((rc = ensure(x.words, (n_from + 4) * sizeof(unsigned)))) return rc;
+  if ((rc = x.room(x.words, (n_from + 4) * sizeof(unsigned)))) return rc;
   hipLaunchKernelGGL(ft_k_cell_parents_write, waves, wave, 0, s->stream, g, ops, n_prog, (unsigned*)x.marks.ptr, parents,
                      (unsigned*)x.words.ptr, totals);
   if ((rc = read_totals(s->stream, x.totals, t))) return rc;
   // a parent's marks start at first word / 8 x 64 and take ceil(words / 8) x 64
-  if ((rc = ensure(x.marks, (n_from / 8 + 1) * 64 * sizeof(unsigned))) ||
-      (rc = ensure(s->cell_progs, (n_cells + 1) * sizeof(int4))) || (rc = ensure(s->cell_shades, (n_cells + 1) * sizeof(int2))))
+  if ((rc = x.room(x.marks, (n_from / 8 + 1) * 64 * sizeof(unsigned))) ||
+      (rc = x.room(s->cell_progs, (n_cells + 1) * sizeof(int4))) || (rc = x.room(s->cell_shades, (n_cells + 1) * sizeof(int2))))
     return rc;
   const unsigned* from = (const unsigned*)x.words.ptr;
   hipLaunchKernelGGL(ft_k_cell_children_count, dim3(n_parents), wave, 0, s->stream, g, ops, (const int2*)parents, from,
@@ -996,7 +1015,7 @@ int build_cell_programs(ft_scene* s, CellScratch& x) {
   const int4 all = make_int4((int)whole[0], (int)whole[1], 2, n_whole);
   const int2 all_shades = make_int2(2 * n_whole, n_prog);
   if ((rc = upload(s->cell_ops, h.cell_ops)) || (rc = upload(s->cell_ext, h.cell_ext)) ||
-      (rc = ensure(s->cell_words, ((size_t)t[0] + cursor + 4) * sizeof(unsigned))))
+      (rc = x.room(s->cell_words, ((size_t)t[0] + cursor + 4) * sizeof(unsigned))))
     return rc;
   // cleared first: the evaluation requests records for the words after a program's last one, so
   // every word has to name a node
@@ -1017,6 +1036,26 @@ int build_cell_programs(ft_scene* s, CellScratch& x) {
   s->dev.cell_ext = (const float4*)s->cell_ext.ptr;
   s->dev.cell_sweep = h.cell_sweep ? 1 : 0;
   return FT_OK;
+}
+
+// Runs one of the builders above.  Cells only speed a scene up: without the memory for them it keeps
+// its program or BVH, and what was allocated for cells that are not used goes back.
+int build_cells(ft_scene* s, CellScratch& x, int (*build)(ft_scene*, CellScratch&)) {
+  const std::string err = g_err;
+  int rc = x.limit ? build(s, x) : FT_OK;
+  if (rc == FT_ERR_OUT_OF_MEMORY) {
+    (void)hipGetLastError();
+    g_err = err;
+    x.drop();
+    rc = FT_OK;
+  }
+  if (s->dev.cells == kCellNone)
+    for (DevBuf* b : {&s->tiny, &s->tiny_boxes, &s->cell_lists, &s->cell_items, &s->leaf_prims, &s->leaf_boxes,
+                      &s->cell_progs, &s->cell_shades, &s->cell_words, &s->cell_ops, &s->cell_ext}) {
+      if (b->ptr) (void)hipFree(b->ptr);
+      *b = DevBuf();
+    }
+  return rc;
 }
 
 }  // namespace
@@ -1108,10 +1147,10 @@ static int create_scene(const ft_scene_ir* ir, uint32_t accel_mode, bool batch_m
     s->plan = fth::plan_emission(h, ir);
     bool emit = !batch_member && (always ? s->plan.any() : (!never && s->plan.any() && fth::emission_pays(h, ir, s->plan)));
     const bool straight = s->straight = emit && s->plan.scene;
-    if (!h.leaf_prims.empty()) rc = build_leaf_lists(s, scratch);
+    if (!h.leaf_prims.empty()) rc = build_cells(s, scratch, build_leaf_lists);
     else if (h.cell_programs && (!straight || (!always && (int)h.prog.size() >= kCellDepthNodes)))
-      rc = build_cell_programs(s, scratch);
-    if (!rc && d.cells == kCellNone && !straight) rc = build_tiny(s);
+      rc = build_cells(s, scratch, build_cell_programs);
+    if (!rc && d.cells == kCellNone && !straight) rc = build_cells(s, scratch, build_tiny);
     if (rc) {
       std::string e = g_err;
       cleanup();

@@ -8,7 +8,8 @@
     primitives, from the smallest tree that gets them; against the emitted straight-line
     scene (FT_EMIT=1, no cells) and against the oracle;
   * tiny scenes: up to the largest and one word past it, against their node program and the oracle;
-  * batches that mix them.
+  * batches that mix them;
+  * the same scenes where there is no memory for cells: the BVH walk and the node program.
 
 Each scene's statistics say that what a test is about does answer its distance.
 """
@@ -377,3 +378,46 @@ def test_batch_of_scene_kinds(kinds, monkeypatch):
     assert np.array_equal(images[0][0], images[1][0])
     # the same arithmetic in differently compiled kernels: a last bit now and then
     assert (np.abs(images[0][1].astype(int) - images[1][1].astype(int)) > 1).mean() <= 1e-3
+
+
+def _scene_of(case):
+    kind, k = case
+    if kind == "parts":
+        return parts_scene(*LIST_CASES[k])
+    if kind == "tree":
+        n, seed, joins, models, plain = TREE_CASES[k]
+        return tree_scene(n, seed, (1.0, 2.0, -6.5), joins, models, plain=plain)
+    text, eye = TINY[k]
+    return CAM % tuple(num(v) for v in eye) + LIGHTS + text
+
+
+WITHOUT_CELLS = [("parts", 1), ("parts", 4)] + [("tree", k) for k in (1, 2, 3, 5, 6)] + [("tiny", k) for k in ("parts4", "spine", "deep")]
+
+
+@pytest.mark.parametrize("case", WITHOUT_CELLS, ids=[f"{a}-{b}" for a, b in WITHOUT_CELLS])
+@pytest.mark.parametrize("mb", ["0", "1"])
+def test_without_memory_for_cells(case, mb, monkeypatch):
+    """FT_CELL_MB: 0 turns cells and tiny words off; with 1 the building of a tree's cells ends at the
+    first allocation beyond it, as where the device has none left (a list of 17 leaves fits).  The scene is
+    created all the same, and nothing that the cells took stays allocated."""
+    import torch
+    monkeypatch.setenv("FT_EMIT", "0")
+    scene = compile_src(_scene_of(case))
+    opts = RenderOptions(width=101, height=67, **OPTS)
+    print(f"[without cells] {case}, {mb} MB", flush=True)
+    for accel in (AccelMode.Bvh, AccelMode.Naive):
+        monkeypatch.setenv("FT_CELL_MB", mb)
+        with GpuScene(scene, accel) as gs:
+            kind = gs.stats().cells
+            if mb == "0" or case[0] == "tree":
+                assert kind == abi.CELLS_NONE
+                against_oracle(scene, accel, gs, opts, str(case))
+    if mb == "1" and case[0] == "tree":
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        held = [GpuScene(scene, AccelMode.Bvh) for _ in range(8)]
+        torch.cuda.synchronize()
+        taken = free - torch.cuda.mem_get_info()[0]
+        for gs in held:
+            gs.close()
+        assert taken < 8 << 22, taken  # the cells' headers alone would be 6 MB a scene
