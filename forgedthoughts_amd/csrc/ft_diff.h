@@ -22,7 +22,8 @@
 
 namespace ftd {
 
-// FLOPs per lane of one tree pass (FMA = 2; add, mul, min, max, abs, compare, sqrt = 1):
+// FLOPs per lane of one pass over the whole tree (what is counted for a pass, though it walks
+// only the words of its point's cell; FMA = 2; add, mul, min, max, abs, compare, sqrt = 1):
 // a sphere leaf translate 3 + length 6 + radius 1, a union_round join 13; a reverse pass
 // adds per sphere 19 (normalised offset, gradient) and per join 22 (partials, child
 // adjoints); one that accumulates parameter gradients adds per sphere 29 (seeded products
@@ -202,7 +203,7 @@ struct DiffEval {
   }
 };
 
-// Adds the FLOPs of `evals` plain passes, `revs` reverse passes and `accs` accumulating
+// Adds the whole-tree FLOPs of `evals` plain passes, `revs` reverse passes and `accs` accumulating
 // reverse passes of this lane to *flops (one atomic per wave).
 __device__ __forceinline__ void diff_count(const DiffArgs& a, unsigned evals, unsigned revs, unsigned accs,
                                           unsigned long long* flops) {
@@ -472,8 +473,8 @@ __device__ __forceinline__ bool diff_item(const DiffArgs& a, int& view, int& til
   return true;
 }
 
-// Forward: t*, s per pixel (t* = -1, s = 0 on a miss).  kCounted adds the work of the
-// image's lanes to *flops.  One wave per block; LDS: the value stacks.
+// Forward: t*, s per pixel (t* = -1, s = 0 on a miss).  kCounted adds the passes of
+// the image's lanes to *flops.  One wave per block; LDS: the value stacks.
 template <bool kCounted>
 __device__ __forceinline__ void diff_forward_body(DiffArgs a, float* __restrict__ t_out, float* __restrict__ s_out,
                                                   unsigned long long* flops) {
@@ -579,7 +580,7 @@ __device__ __forceinline__ bool interior_hit(const float* __restrict__ t, int w,
 
 // Adjoint: accumulates sum over pixels of dL/dth into per-block partial sums (FP64): one wave
 // per block, kDiffTiles tiles one after the other, so a block's sums are added in a fixed order.
-// kCounted adds the work of the lanes with a non-zero upstream gradient to *flops.
+// kCounted adds the passes of the lanes with a non-zero upstream gradient to *flops.
 // LDS: gradient accumulator [n_params doubles], value stacks, kept operands.
 constexpr int kDiffTiles = 4;
 template <bool kCounted>

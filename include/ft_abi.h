@@ -544,11 +544,13 @@ int ft_diff_loss_grad(ft_diff* diff, float w_t, float w_s, double* loss_out, dou
 /* `steps` Adam steps on the device (beta1 0.9, beta2 0.999, eps 1e-8); losses_out
  * (nullable) receives L before each step.  Synchronous. */
 int ft_diff_fit(ft_diff* diff, uint32_t steps, float lr, float w_t, float w_s, double* losses_out);
-/* sdf_flops: FLOPs of the forward and adjoint tree passes since counting was turned on
- * (FLOP counting on), else 0. */
+/* sdf_flops: FLOPs of the forward and adjoint passes since counting was turned on (FLOP
+ * counting on), else 0: each pass priced as a walk of the whole tree, though the kernels walk
+ * what a point's cell keeps of it, so that it measures the passes a step needs and not the
+ * rate of the arithmetic. */
 int ft_diff_stats(ft_diff* diff, ft_render_stats* out);
 /* Turns FLOP counting on (1, clears the counter) or off (0): later forwards and adjoints run
- * the *_counted kernels, which add their per-lane tree-pass FLOPs with one atomic per wave. */
+ * the *_counted kernels, which add their lanes' passes with one atomic per wave. */
 int ft_diff_set_flop_counting(ft_diff* diff, int enable);
 
 /* Scene specialisation diagnostics (no GPU needed).  ft_emit_scene_source writes the
