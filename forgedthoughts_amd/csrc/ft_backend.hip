@@ -178,11 +178,13 @@ const LaunchCfg& cfg_of(const ft_scene* s, int k) { return s->cfg[k == fth::kRtc
 uint32_t mod_key(int k, bool counted, const LaunchCfg& c) {
   return (uint32_t)k | (counted ? 1u << 4 : 0u) | (c.wpe << 8) | (c.unroll << 12) | (c.shade_inline << 16);
 }
+// Kernel k runs the scene's emitted code: the depth kernel of a scene with cell programs has none.
+bool runs_emitted(const ft_scene* s, int k) {
+  return !s->source.empty() && !(k == fth::kRtcDepth && s->dev.cells == kCellPrograms);
+}
 // Kernel k of shape c runs from a runtime-compiled code object (else the precompiled one).
-// (The depth kernel of a scene with cell programs runs none of the scene's emitted code.)
 bool needs_module(const ft_scene* s, int k, bool counted, const LaunchCfg& c) {
-  const bool emitted = !s->source.empty() && !(k == fth::kRtcDepth && s->dev.cells == kCellPrograms);
-  return counted || emitted || !c.default_code() || fth::strict_math();
+  return counted || runs_emitted(s, k) || !c.default_code() || fth::strict_math();
 }
 hipFunction_t module_function(const ft_scene* s, int k, bool counted, const LaunchCfg& c) {
   auto it = s->mods.find(mod_key(k, counted, c));
@@ -201,12 +203,13 @@ int load_module(ft_scene* s, int k, bool counted, const LaunchCfg& c, const std:
   return publish_module(s, m);
 }
 
-std::string module_source(const ft_scene* s, bool counted) {
+std::string module_source(const ft_scene* s, int k, bool counted) {
+  const bool emitted = runs_emitted(s, k);
   // tiny scenes keep no operation counts: their counted kernels run the program
-  const bool none = (!s->source.empty() && s->plan.scene) || (counted && s->dev.cells == kCellTiny);
+  const bool none = (emitted && s->plan.scene) || (counted && s->dev.cells == kCellTiny);
   const int mode = none ? kCellNone : s->dev.cells;
   return "#define FT_SCENE_MODE " + std::to_string(mode) + "\n" +
-         (s->source.empty() ? std::string("#include \"ft_kernels.h\"\n") : s->source);
+         (emitted ? s->source : std::string("#include \"ft_kernels.h\"\n"));
 }
 
 // Builds and loads the code object kernel `k` needs under shape `c` (no-op when it runs
@@ -218,7 +221,7 @@ int prepare(ft_scene* s, int k, const LaunchCfg& c) {
   std::vector<char> code;
   std::string err;
   double ms = 0.0;
-  if (!fth::rtc_compile(module_source(s, counted), k, counted, (int)c.wpe, (int)c.unroll, (int)c.shade_inline, code, ms, err))
+  if (!fth::rtc_compile(module_source(s, k, counted), k, counted, (int)c.wpe, (int)c.unroll, (int)c.shade_inline, code, ms, err))
     return fail(FT_ERR_COMPILE_FAILED, err);
   s->compile_ms += ms;
   return load_module(s, k, counted, c, code);
@@ -586,7 +589,7 @@ bool tune_cache_get(uint64_t key, uint32_t kind, LaunchCfg& c) {
     return true;
   }
   char name[48];
-  std::snprintf(name, sizeof(name), "tune6_%016llx.txt", (unsigned long long)key);
+  std::snprintf(name, sizeof(name), "tune7_%016llx.txt", (unsigned long long)key);
   const std::string path = fth::cache_file(name);
   if (path.empty()) return false;
   FILE* f = std::fopen(path.c_str(), "r");
@@ -606,7 +609,7 @@ void tune_cache_put(uint64_t key, const LaunchCfg& c) {
   std::lock_guard<std::mutex> lk(g_tune_mu);
   g_tune_cache[key] = c;
   char name[48];
-  std::snprintf(name, sizeof(name), "tune6_%016llx.txt", (unsigned long long)key);
+  std::snprintf(name, sizeof(name), "tune7_%016llx.txt", (unsigned long long)key);
   const std::string path = fth::cache_file(name);
   if (path.empty()) return;
   const std::string tmp = path + ".tmp";
@@ -639,7 +642,7 @@ int build_variants(ft_scene* s, int k, const std::vector<LaunchCfg>& variants) {
   std::vector<std::string> errs(variants.size());
   std::vector<double> ms(variants.size(), 0.0);
   std::vector<char> ok(variants.size(), 1), need(variants.size(), 0);
-  const std::string src = module_source(s, false);
+  const std::string src = module_source(s, k, false);
   std::vector<std::thread> th;
   for (size_t i = 0; i < variants.size(); ++i) {
     if (!needs_module(s, k, false, variants[i]) || module_function(s, k, false, variants[i])) continue;

@@ -421,3 +421,26 @@ def test_without_memory_for_cells(case, mb, monkeypatch):
         for gs in held:
             gs.close()
         assert taken < 8 << 22, taken  # the cells' headers alone would be 6 MB a scene
+
+
+def test_depth_kernels_of_other_shapes_run_the_cells(monkeypatch):
+    """A tree whose depth comes from cells and whose Whitted frame is straight-line code (63 nodes): the
+    depth kernels built for a launch shape of their own, and the counted ones, run the cells too.  They
+    count what the same scene counts without emission (before, all 63 nodes at every point)."""
+    scene = compile_src(tree_scene(32, 9, (1.0, 2.0, -6.5), JOINS[:4], plain=True))
+    opts = RenderOptions(width=101, height=67, **OPTS)
+    counts, images = [], []
+    for emit in ("auto", "0"):
+        monkeypatch.setenv("FT_EMIT", emit)
+        with GpuScene(scene, AccelMode.Bvh) as gs:
+            assert gs.stats().cells == abi.CELLS_PROGRAMS
+            assert gs.stats().flags == (abi.STATS_EMITTED_SCENE if emit == "auto" else 0)
+            images.append(gs.render_depth(opts, 1))
+            gs.set_launch_config(0, block_waves=1, tile_width=8, waves_per_eu=4, march_unroll=2, shade_inline=0)
+            images.append(gs.render_depth(opts, 1))
+            gs.set_flop_counting(True)
+            images.append(gs.render_depth(opts, 1))
+            counts.append(gs.stats().sdf_flops)
+    assert counts[0] == counts[1] > 0
+    for got in images[1:]:
+        same_depth(got, images[0], "another shape")
