@@ -1889,6 +1889,8 @@ int ft_batch_set_flop_counting(ft_batch* b, int enable) {
   for (ft_scene* s : b->scenes) {
     s->dev.flops = enable ? (unsigned long long*)b->flops.ptr : nullptr;
     s->dev.atlas_samples = enable ? (unsigned long long*)b->flops.ptr + 1 : nullptr;
+    // tiny scenes keep no counts: while counting they run the program (module_source)
+    if (s->dev.tiny) s->dev.cells = enable ? kCellNone : kCellTiny;
     if ((rc = publish(s))) return rc;
   }
   b->counting = enable != 0;

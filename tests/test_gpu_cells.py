@@ -444,3 +444,34 @@ def test_depth_kernels_of_other_shapes_run_the_cells(monkeypatch):
     assert counts[0] == counts[1] > 0
     for got in images[1:]:
         same_depth(got, images[0], "another shape")
+
+
+def test_batches_count_tiny_scenes():
+    """The FLOPs of a batch's tiny scene are those of the scene alone, seen the same way; images with and
+    without counting are the same."""
+    import torch
+    from forgedthoughts_amd.render import GpuBatch
+    text, eye = TINY["parts4"]
+    scene = compile_src(LIGHTS + text)
+    opts = RenderOptions(width=61, height=37, **OPTS)
+    with GpuScene(with_camera(scene, eye, (0.0, 0.0, 0.0), 50.0), AccelMode.Bvh) as gs:
+        assert gs.stats().cells == abi.CELLS_TINY
+        gs.set_flop_counting(True)
+        gs.render_depth(opts, 1)
+        want = gs.stats().sdf_flops
+    views = GpuBatch.views([(0, eye, (0.0, 0.0, 0.0), 50.0)])
+    images = []
+    with GpuBatch([scene]) as b:
+        for counting in (False, True, False):
+            for flags in (0, abi.BATCH_SEPARATE):
+                b.set_flop_counting(counting)
+                d = torch.zeros(61 * 37 * 3, dtype=torch.uint8, device="cuda")
+                b.render_device(views, opts, RaySettings(1, 64, 1), abi.BATCH_DEPTH | flags, d.data_ptr(), 0)
+                b.synchronize()
+                images.append(d.cpu().numpy())
+                if counting:
+                    assert abs(b.stats().sdf_flops - want) <= 0.02 * want, (b.stats().sdf_flops, want)
+    assert want > 0 and images[0].any()
+    for got in images[1:]:
+        # the program's distances agree with the words' to the last bits: a step of the image at most
+        assert (np.abs(got.astype(int) - images[0].astype(int)) <= 1).all()
