@@ -122,6 +122,8 @@ struct ft_scene {
   // scene specialisation
   fth::EmitPlan plan;
   bool straight = false;  // emitted, and a scene whose distance straight-line code can be (cells may answer it instead)
+  float cell_gain = 0.0f;       // cell programs: the tree's nodes for each word of a cell on the surface
+  bool depth_straight = false;  // of the depth call at hand, for a scene with both (choose_depth)
   std::string source;                              // emitted translation unit (empty: interpreter)
   // runtime-compiled code objects, one per (kernel, counted, occupancy, unroll), built on
   // first use: the scene-specialised kernels, the *_counted variants (FLOP counting on) and
@@ -175,19 +177,20 @@ const void* const kKernelStubs[fth::kRtcKernelCount] = {(const void*)ft_k_depth,
                                                         (const void*)ft_k_whitted_48, (const void*)ft_k_whitted_128};
 
 const LaunchCfg& cfg_of(const ft_scene* s, int k) { return s->cfg[k == fth::kRtcDepth ? 0 : 1]; }
-uint32_t mod_key(int k, bool counted, const LaunchCfg& c) {
-  return (uint32_t)k | (counted ? 1u << 4 : 0u) | (c.wpe << 8) | (c.unroll << 12) | (c.shade_inline << 16);
+uint32_t mod_key(int k, bool counted, bool emitted, const LaunchCfg& c) {
+  return (uint32_t)k | (counted ? 1u << 4 : 0u) | (emitted ? 1u << 5 : 0u) | (c.wpe << 8) | (c.unroll << 12) | (c.shade_inline << 16);
 }
-// Kernel k runs the scene's emitted code: the depth kernel of a scene with cell programs has none.
+// Kernel k runs the scene's emitted code: the depth kernel of a scene with cell programs has none,
+// but for the calls that straight-line code serves better.
 bool runs_emitted(const ft_scene* s, int k) {
-  return !s->source.empty() && !(k == fth::kRtcDepth && s->dev.cells == kCellPrograms);
+  return !s->source.empty() && !(k == fth::kRtcDepth && s->dev.cells == kCellPrograms && !s->depth_straight);
 }
 // Kernel k of shape c runs from a runtime-compiled code object (else the precompiled one).
 bool needs_module(const ft_scene* s, int k, bool counted, const LaunchCfg& c) {
   return counted || runs_emitted(s, k) || !c.default_code() || fth::strict_math();
 }
 hipFunction_t module_function(const ft_scene* s, int k, bool counted, const LaunchCfg& c) {
-  auto it = s->mods.find(mod_key(k, counted, c));
+  auto it = s->mods.find(mod_key(k, counted, runs_emitted(s, k), c));
   return it == s->mods.end() ? nullptr : it->second.second;
 }
 
@@ -199,7 +202,7 @@ int load_module(ft_scene* s, int k, bool counted, const LaunchCfg& c, const std:
   const std::string name = std::string(kKernelNames[k]) + (counted ? "_counted" : "");
   hipFunction_t f = nullptr;
   FT_HIP(hipModuleGetFunction(&f, m, name.c_str()));
-  s->mods[mod_key(k, counted, c)] = {m, f};
+  s->mods[mod_key(k, counted, runs_emitted(s, k), c)] = {m, f};
   return publish_module(s, m);
 }
 
@@ -316,6 +319,35 @@ int clear_flops(ft_scene* s) {
   return FT_OK;
 }
 
+// Straight-line code or cell programs, for a tree that could have either.  The first costs what the
+// tree has, the second what a cell on the surface keeps, so the line lies at the nodes of the tree for
+// each word of such a cell (cell_gain), and the lower the more waves a launch has to hide the loads of
+// the cells behind.  Straight-line against cells by gain, trees of 24 to 400 spread, dense, packed or of
+// mixed operators (depth previews, then Whitted frames of 1 sample at 96x96 and 4 at 640x360; above 1
+// the cells are the faster):
+//   gain   96x96  256x256  512x512  800x800  1200x1200   96x96   640x360
+//   7..9   0.4    -        -        -        -           0.5     0.7
+//   11     0.57   0.76     0.75     0.94     1.19        0.6     0.6
+//   12-13  0.65   0.9      1.15     1.3      1.4         0.73    1.0
+//   14     0.83   0.9      0.8-1.2  1.2      1.4         0.8     1.0
+//   16     0.9    1.06     1.2      1.4      1.7         0.83    1.2
+//   18-20  1.1    1.1      1.5      1.7      1.7         1.0     1.5
+//   24     1.2    1.2      1.2      1.4      1.6         1.2     1.4
+//   37-46  2      2.2      -        2.3      -           2.2     2.5
+// A depth preview takes whichever suits its launch; the Whitted kernels, seconds to compile, are one
+// of the two for good.  Trees of fewer than kCellTreeNodes nodes do not come near (a spread one of 28,
+// 55 nodes: 11), and the building of their cells (about a millisecond) is spared.
+constexpr int kCellTreeNodes = 57;
+constexpr float kCellGainSmall = 18.0f, kCellGainMiddle = 15.0f, kCellGainLarge = 11.0f;
+constexpr uint64_t kCellMiddleWaves = 4096, kCellLargeWaves = 16384;
+
+// Decides what a depth launch over the camera's rows runs, where the scene has both (before prepare).
+void choose_depth(ft_scene* s, const CamArgs& cam) {
+  const uint64_t waves = ((uint64_t)cam.width * cam.rows + 63) / 64;
+  const float line = waves >= kCellLargeWaves ? kCellGainLarge : (waves >= kCellMiddleWaves ? kCellGainMiddle : kCellGainSmall);
+  s->depth_straight = s->straight && s->plan.scene && s->dev.cells == kCellPrograms && s->cell_gain < line;
+}
+
 // Enqueues the depth preview of the camera's rows (the kernel must be prepared).
 int depth_enqueue(ft_scene* s, const CamArgs& cam_in, const TraceParams& tp_in, unsigned char* rgb_dev, float* t_dev) {
   CamArgs cam = cam_in;
@@ -339,6 +371,7 @@ int depth_impl(ft_scene* s, const ft_render_options* o, uint32_t aa, unsigned ch
   CamArgs cam = make_cam(s, *o, aa, s->cfg[0].tile_w);
   TraceParams tp = make_tp(*o, 1);
   FT_HIP(hipSetDevice(s->device));
+  choose_depth(s, cam);
   if ((rc = prepare(s, fth::kRtcDepth))) return rc;  // compile outside the timed region
   return depth_enqueue(s, cam, tp, rgb_dev, t_dev);
 }
@@ -526,8 +559,10 @@ int progressive_impl(ft_scene* s, bool whitted, const ft_render_options* o, cons
   const size_t W = o->width, H = o->height;
   if ((rc = ensure(s->rgb, W * H * 3))) return rc;
   FT_HIP(hipSetDevice(s->device));
-  if ((rc = prepare(s, kernel))) return rc;
   const uint32_t ts = std::max<uint32_t>(tile_size, 1u);
+  cam.rows = (int)std::min<size_t>(ts, H);
+  choose_depth(s, cam);
+  if ((rc = prepare(s, kernel))) return rc;
   const uint32_t tiles_x = (uint32_t)((W + ts - 1) / ts), tiles_y = (uint32_t)((H + ts - 1) / ts);
   std::vector<uint8_t> image(W * H * 3, 0);
   ft_progress pg{};
@@ -681,8 +716,9 @@ int autotune_impl(ft_scene* s, uint32_t kind, const ft_render_options* o, const 
   if (kind == FT_KIND_WHITTED && !(flags & FT_TUNE_FULL) && rs.aa_samples > 16) rs.aa_samples = 16;
   if ((rc = ensure(s->rgb, (size_t)o->width * o->height * 3))) return rc;
   int k = fth::kRtcDepth;
+  CamArgs cam = make_cam(s, *o, rs.aa_samples);
+  choose_depth(s, cam);
   if (kind == FT_KIND_WHITTED) {
-    CamArgs cam;
     TraceParams tp;
     if ((rc = whitted_check(s, o, &rs, cam, tp, k))) return rc;
   }
@@ -775,9 +811,9 @@ struct CellScratch {
     return bytes > limit ? fail(FT_ERR_OUT_OF_MEMORY, "cells larger than FT_CELL_MB") : ensure(b, bytes);
   }
   int reset() {
-    int rc = ensure(totals, 2 * sizeof(CellTotal));
+    int rc = ensure(totals, kCellTotals * sizeof(CellTotal));
     if (rc) return rc;
-    FT_HIP(hipMemset(totals.ptr, 0, 2 * sizeof(CellTotal)));
+    FT_HIP(hipMemset(totals.ptr, 0, kCellTotals * sizeof(CellTotal)));
     FT_HIP(hipStreamSynchronize(nullptr));
     return FT_OK;
   }
@@ -794,12 +830,6 @@ static int create_scene(const ft_scene_ir* ir, uint32_t accel_mode, bool batch_m
 
 // ------------------------------------------------------------------ cells
 namespace {
-
-// Straight-line code or cell programs, for a scene that could have either, by the nodes of its
-// program.  Straight-line against cells: previews at 1280x720 0.17 / 0.38 ms at 8 primitives (15
-// nodes), 0.47 / 0.51 at 24, 0.77 / 0.65 at 32, 1.73 / 0.84 at 64; 4-bounce Whitted at 1280x720
-// and 4 samples 0.8 / 1.3 ms at 8, 4.5 / 6.4 at 32, 7.0 / 7.8 at 48, 9.4 / 5.8 at 64.
-constexpr int kCellDepthNodes = 57, kCellWhittedNodes = 111;
 
 CellGrid cell_grid(const fth::HostScene& h) {
   CellGrid g;
@@ -824,8 +854,8 @@ void set_grid(DevScene& d, const fth::HostScene& h, int kind) {
 }
 
 // The counters of a count / write pair of launches: read and cleared in between.
-int read_totals(hipStream_t stream, DevBuf& totals, CellTotal t[2]) {
-  const CellTotal zero[2] = {0, 0};
+int read_totals(hipStream_t stream, DevBuf& totals, CellTotal t[kCellTotals]) {
+  const CellTotal zero[kCellTotals] = {};
   FT_HIP(hipGetLastError());
   FT_HIP(hipStreamSynchronize(stream));
   FT_HIP(hipMemcpy(t, totals.ptr, sizeof(zero), hipMemcpyDeviceToHost));
@@ -846,7 +876,7 @@ int build_leaf_lists(ft_scene* s, CellScratch& x) {
   const dim3 waves((unsigned)((n_parents + 63) / 64)), wave(64);
   const float4* prims = (const float4*)s->leaf_prims.ptr;
   const float4* boxes = (const float4*)s->leaf_boxes.ptr;
-  CellTotal t[2];
+  CellTotal t[kCellTotals];
   if ((rc = x.reset()) || (rc = x.room(x.parents, (size_t)n_parents * sizeof(int4)))) return rc;
   CellTotal* totals = (CellTotal*)x.totals.ptr;
   hipLaunchKernelGGL(ft_k_leaf_parents_count, waves, wave, 0, s->stream, g, prims, boxes, np, n, (int4*)x.parents.ptr, totals);
@@ -971,7 +1001,7 @@ int build_cell_programs(ft_scene* s, CellScratch& x) {
   const dim3 waves((unsigned)((n_parents + 63) / 64)), wave(64);
   const DOp* ops = (const DOp*)s->ops.ptr;
   int rc;
-  CellTotal t[2];
+  CellTotal t[kCellTotals];
   if ((rc = x.reset()) || (rc = x.room(x.parents, (size_t)n_parents * sizeof(int2))) ||
       (rc = x.room(x.marks, (size_t)((n_prog + 7) / 8) * n_parents * sizeof(unsigned))))
     return rc;
@@ -993,6 +1023,9 @@ int build_cell_programs(ft_scene* s, CellScratch& x) {
   hipLaunchKernelGGL(ft_k_cell_children_count, dim3(n_parents), wave, 0, s->stream, g, ops, (const int2*)parents, from,
                      (unsigned*)x.marks.ptr, (int4*)s->cell_progs.ptr, (int2*)s->cell_shades.ptr, totals);
   if ((rc = read_totals(s->stream, x.totals, t))) return rc;
+  const double kept = t[3] ? (double)t[2] / (double)t[3] : (double)t[1] / (double)n_cells;
+  s->cell_gain = (float)((double)n_prog / std::max(kept, 1.0));
+  if (s->straight && s->cell_gain < kCellGainLarge) return FT_OK;
   if ((double)t[1] > 0.25 * (double)n_prog * (double)n_cells || t[0] + 4ull * n_prog > (1u << 31)) return FT_OK;
   // the whole program in front, then the cells', and room to read ahead at the end
   std::vector<unsigned> whole;
@@ -1151,7 +1184,7 @@ static int create_scene(const ft_scene_ir* ir, uint32_t accel_mode, bool batch_m
     bool emit = !batch_member && (always ? s->plan.any() : (!never && s->plan.any() && fth::emission_pays(h, ir, s->plan)));
     const bool straight = s->straight = emit && s->plan.scene;
     if (!h.leaf_prims.empty()) rc = build_cells(s, scratch, build_leaf_lists);
-    else if (h.cell_programs && (!straight || (!always && (int)h.prog.size() >= kCellDepthNodes)))
+    else if (h.cell_programs && (!straight || (!always && (int)h.prog.size() >= kCellTreeNodes)))
       rc = build_cells(s, scratch, build_cell_programs);
     if (!rc && d.cells == kCellNone && !straight) rc = build_cells(s, scratch, build_tiny);
     if (rc) {
@@ -1159,7 +1192,7 @@ static int create_scene(const ft_scene_ir* ir, uint32_t accel_mode, bool batch_m
       cleanup();
       return fail(rc, e);
     }
-    if (straight && d.cells == kCellPrograms && (int)h.prog.size() >= kCellWhittedNodes) {
+    if (straight && d.cells == kCellPrograms && s->cell_gain >= kCellGainSmall) {
       // the sweep is still worth compiling where the cells' shading words do not serve
       s->plan.scene = false;
       s->plan.sweep = s->plan.sweep && !d.cell_sweep;

@@ -475,9 +475,10 @@ __device__ __forceinline__ float3 child_centre(const CellGrid& g, int i, int lan
   return cell_centre(g, g.cell, x, y, z);
 }
 
-// The counters of a build, [0] words and [1] what the host decides by beside them.  They hold
+// The counters of a build, [0] words and the others what the host decides by beside them.  They hold
 // more than 32 bits: whether a build's words fit is decided from their whole count.
 typedef unsigned long long CellTotal;
+constexpr int kCellTotals = 4;
 // A leaf list has at most this many entries of a kind, since its two counts share a word; scenes
 // with longer ones keep the BVH walk.
 constexpr int kLongestList = 0x7fff;
@@ -666,11 +667,12 @@ __device__ __forceinline__ float3 join_one_interval(int kind, const DOp& o, bool
 
 // `words`: null for the scene program (n words), else its shading words.  `marks`: this lane's
 // first mark word, `stride` words apart.  Counting (kWrite = false) sets r.w and sh.y; writing
-// takes the room given in r.z and sh.x (kShades only: shading words alone).
+// takes the room given in r.z and sh.x (kShades only: shading words alone).  `surface`, of counting:
+// the cell may hold some of the surface.
 template <bool kWrite, bool kShadesOnly>
 __device__ __forceinline__ void cell_program(const DOp* __restrict__ ops_, const unsigned* __restrict__ words_, int n,
                                              float3 c, float R, float margin, bool mine, unsigned* __restrict__ marks,
-                                             int stride, int4& r, int2& sh, unsigned* __restrict__ out) {
+                                             int stride, int4& r, int2& sh, unsigned* __restrict__ out, bool& surface) {
   const auto ops = uniform_ptr(ops_);
   const auto words = uniform_ptr(words_);
   auto word = [&](int k) { return words_ ? words[k] : (unsigned)k; };
@@ -708,6 +710,7 @@ __device__ __forceinline__ void cell_program(const DOp* __restrict__ ops_, const
         bits = 0u;
       }
     }
+    surface = lo[0] <= 0.0f && hi[0] >= 0.0f;  // the root's interval
     __threadfence_block();
   }
   // from the root down (reverse post order): a bit per pending subtree, set where it remains;
@@ -779,13 +782,15 @@ __device__ __forceinline__ void cell_parents_body(CellGrid g, const DOp* __restr
   const int m = min(i, n_parents - 1);
   int4 r = make_int4(0, 0, 0, 0);
   int2 sh = kWrite ? parents[m] : make_int2(0, 0);
+  bool surface = false;
   if (kWrite) sh.x = (int)take_room(&totals[0], mine ? (unsigned)(sh.y + 7) & ~7u : 0u);
   cell_program<kWrite, true>(ops, nullptr, n_prog, parent_centre(g, m), cell_radius(g, g.cell * kCellChildren),
-                             0.25f * g.margin, mine, marks + m, n_parents, r, sh, words);
+                             0.25f * g.margin, mine, marks + m, n_parents, r, sh, words, surface);
   if (mine) parents[m] = sh;
   if (!kWrite && mine) atomicAdd(&totals[0], (CellTotal)((unsigned)(sh.y + 7) & ~7u));
 }
-// Children (a wave per parent).  totals[0]: words, [1]: distance words alone.
+// Children (a wave per parent).  totals[0]: words, [1]: distance words alone, [2]: those of the cells on
+// the surface, [3]: these cells.
 template <bool kWrite>
 __device__ __forceinline__ void cell_children_body(CellGrid g, const DOp* __restrict__ ops, const int2* __restrict__ parents,
                                                    const unsigned* __restrict__ parent_words, unsigned* __restrict__ marks,
@@ -801,15 +806,20 @@ __device__ __forceinline__ void cell_children_body(CellGrid g, const DOp* __rest
     r.z = (int)take_room(&totals[0], (unsigned)(2 * (r.w - 1) + ((sh.y + 1) & ~1)));
     sh.x = r.z + 2 * (r.w - 1);
   }
+  bool surface = false;
   // the parent's marks: 64 lanes of ceil(n / 8) words, placed by its first word
   unsigned* const m = marks + (size_t)(from.x / 8) * 64 + threadIdx.x;
   cell_program<kWrite, false>(ops, parent_words + from.x, from.y, c, cell_radius(g, g.cell), 0.25f * g.margin, true, m, 64,
-                              r, sh, words);
+                              r, sh, words, surface);
   progs[index] = r;
   shades[index] = sh;
   if (!kWrite) {
     atomicAdd(&totals[0], (CellTotal)(2 * (r.w - 1) + ((sh.y + 1) & ~1)));
     atomicAdd(&totals[1], (CellTotal)r.w);
+    if (surface) {
+      atomicAdd(&totals[2], (CellTotal)r.w);
+      atomicAdd(&totals[3], (CellTotal)1);
+    }
   }
 }
 

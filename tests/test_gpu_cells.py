@@ -423,27 +423,55 @@ def test_without_memory_for_cells(case, mb, monkeypatch):
         assert taken < 8 << 22, taken  # the cells' headers alone would be 6 MB a scene
 
 
-def test_depth_kernels_of_other_shapes_run_the_cells(monkeypatch):
-    """A tree whose depth comes from cells and whose Whitted frame is straight-line code (63 nodes): the
-    depth kernels built for a launch shape of their own, and the counted ones, run the cells too.  They
-    count what the same scene counts without emission (before, all 63 nodes at every point)."""
-    scene = compile_src(tree_scene(32, 9, (1.0, 2.0, -6.5), JOINS[:4], plain=True))
-    opts = RenderOptions(width=101, height=67, **OPTS)
-    counts, images = [], []
-    for emit in ("auto", "0"):
+# nodes of the tree for each word of a cell on the surface: 7 of the 63, 14 of the 95, 20 of the 127
+GAINS = {"packed": (32, 1, JOINS[:1], 1.2), "dense": (48, 1, JOINS[:1], 2.5), "operators": (64, 1, JOINS[:4], 2.5)}
+
+
+@pytest.mark.parametrize("case", list(GAINS))
+def test_straight_line_code_or_cells(case, monkeypatch):
+    """Which of the two gives a tree's depth: straight-line code, cells in large launches, cells.  The counted
+    kernels, and those built for a launch shape of their own, run what the ordinary ones run: they count
+    the tree's nodes at every point or the words of its cell."""
+    n, seed, joins, extent = GAINS[case]
+    scene = compile_src(tree_scene(n, seed, (1.0, 2.0, -6.5), joins, extent=extent, plain=True))
+    sizes = {"small": (101, 67), "large": (1024, 1024)}
+    counts, images = {}, {}
+    for emit in ("auto", "0", "1"):
         monkeypatch.setenv("FT_EMIT", emit)
         with GpuScene(scene, AccelMode.Bvh) as gs:
-            assert gs.stats().cells == abi.CELLS_PROGRAMS
-            assert gs.stats().flags == (abi.STATS_EMITTED_SCENE if emit == "auto" else 0)
-            images.append(gs.render_depth(opts, 1))
-            gs.set_launch_config(0, block_waves=1, tile_width=8, waves_per_eu=4, march_unroll=2, shade_inline=0)
-            images.append(gs.render_depth(opts, 1))
-            gs.set_flop_counting(True)
-            images.append(gs.render_depth(opts, 1))
-            counts.append(gs.stats().sdf_flops)
-    assert counts[0] == counts[1] > 0
-    for got in images[1:]:
-        same_depth(got, images[0], "another shape")
+            print(f"[straight or cells] {case} FT_EMIT={emit}", flush=True)
+            if emit == "auto":
+                assert gs.stats().cells == (abi.CELLS_NONE if case == "packed" else abi.CELLS_PROGRAMS)
+                assert gs.stats().flags == (0 if case == "operators" else abi.STATS_EMITTED_SCENE)
+            for size, (w, h) in sizes.items():
+                opts = RenderOptions(width=w, height=h, **OPTS)
+                images[emit, size] = gs.render_depth(opts, 1)
+                if size == "small":
+                    gs.set_launch_config(abi.KIND_DEPTH, march_unroll=2)
+                    same_depth(gs.render_depth(opts, 1), images[emit, size], "another shape")
+                    gs.set_launch_config(abi.KIND_DEPTH)
+                gs.set_flop_counting(True)
+                same_depth(gs.render_depth(opts, 1), images[emit, size], "counted")
+                counts[emit, size] = gs.stats().sdf_flops
+                gs.set_flop_counting(False)
+                same_depth(gs.render_depth(opts, 1), images[emit, size], "again")
+    for size in sizes:
+        same_depth(images["0", size], images["1", size], "straight-line code against cells")
+        assert 0 < 2 * counts["0", size] < counts["1", size]
+        straight = case == "packed" or (case == "dense" and size == "small")
+        assert counts["auto", size] == counts["1" if straight else "0", size]
+    # rows of 64 are a small launch each, one tile row of the whole image is a large one
+    if case == "dense":
+        monkeypatch.setenv("FT_EMIT", "auto")
+        with GpuScene(scene, AccelMode.Bvh) as gs:
+            for tile, size in ((64, "small"), (1024, "large")):
+                opts = RenderOptions(width=1024, height=1024, **OPTS)
+                gs.set_flop_counting(True)
+                rgb = gs.render_depth_progressive(opts, 1, tile, lambda progress, image: False)
+                total = gs.stats().sdf_flops
+                gs.set_flop_counting(False)
+                assert total == counts["1" if size == "small" else "0", "large"]
+                assert (np.abs(rgb.astype(int) - images["0", "large"][0].astype(int)) > 1).sum() <= 600
 
 
 def test_batches_count_tiny_scenes():
