@@ -909,7 +909,11 @@ int build_leaf_lists(ft_scene* s, CellScratch& x) {
 // Tiny against the node program / BVH walk it replaces (96x96 preview, 1280x720 Whitted at 4
 // samples, ms): 1 part 0.16 / 0.20 and 1.44 / 1.59, 4 parts 0.31 / 0.46 and 1.76 / 2.17,
 // 7 parts 0.38 / 0.44 and 1.96 / 2.19, a blend of 4 0.33 / 0.57 and 1.79 / 2.38, of 7
-// 0.61 / 0.66 and 2.63 / 2.78: beyond kTinyWords words the advantage is gone.
+// 0.61 / 0.66 and 2.63 / 2.78: beyond kTinyWords words the advantage is gone.  A rotated or shelled part
+// is evaluated from its record, which costs as much as in the program, and the BVH leaves out
+// distant ones: eight such parts spread out (640x360: preview 1.01 / 0.88, Whitted 1.36 / 1.13), six
+// 0.79 / 0.71 and 1.07 / 1.01, four 0.44 / 0.47 and 0.61 / 0.70, so four are the most.
+constexpr size_t kTinyExtended = 4;
 int build_tiny(ft_scene* s, CellScratch&) {
   const fth::HostScene& h = s->host;
   const int n_prog = (int)h.prog.size(), n_leaves = (int)h.leaves.size();
@@ -980,6 +984,8 @@ int build_tiny(ft_scene* s, CellScratch&) {
     boxes.push_back({{L.bmin[0], L.bmin[1], L.bmin[2]}, order[i], {L.bmax[0], L.bmax[1], L.bmax[2]}, rank[order[i]]});
   }
   if (words.size() > (size_t)kTinyWords) return FT_OK;
+  const size_t extended = (size_t)std::count_if(words.begin(), words.end(), [](const DTiny& w) { return (w.flags & kWordExtended) != 0u; });
+  if (!naive && n_leaves > 1 && extended > kTinyExtended) return FT_OK;
   s->dev.n_tiny = (int)words.size();
   words.resize(kTinyWords);  // the first kTinyHeld are read whatever the count
   boxes.resize(kTinyWords);
