@@ -2021,9 +2021,12 @@ unsigned diff_waves(const ft_diff* d) {
 unsigned diff_blocks(const ft_diff* d) { return (diff_waves(d) + kDiffTiles - 1) / kDiffTiles; }  // of the adjoint
 size_t diff_pixels(const ft_diff* d) { return (size_t)d->n_views * d->opts.width * d->opts.height; }
 
+void diff_build_cells(ft_diff* d) {
+  hipLaunchKernelGGL(ft_k_diff_cells, dim3((unsigned)((kDiffCellCount + 63) / 64)), dim3(64), 0, d->stream, diff_args(d));
+}
 int diff_forward_enqueue(ft_diff* d) {
   const DiffArgs a = diff_args(d);
-  hipLaunchKernelGGL(ft_k_diff_cells, dim3((unsigned)((kDiffCellCount + 63) / 64)), dim3(64), 0, d->stream, a);
+  if (d->n_prims > 1) diff_build_cells(d);  // one sphere's cells all hold it, whatever its parameters
   if (d->counting)
     hipLaunchKernelGGL(ft_k_diff_forward_counted, dim3(diff_waves(d)), dim3(64), 0, d->stream, a, (float*)d->t.ptr,
                        (float*)d->s.ptr, (unsigned long long*)d->flops.ptr);
@@ -2156,6 +2159,13 @@ int ft_diff_create(uint32_t n_prims, const ft_view* views, uint32_t n_views, con
     g_err = "clearing the cell words failed";
     return bail(FT_ERR_LAUNCH_FAILED);
   }
+  if (n_prims == 1) {
+    diff_build_cells(d);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(d->stream) != hipSuccess) {
+      g_err = "building the cells failed";
+      return bail(FT_ERR_LAUNCH_FAILED);
+    }
+  }
   if (diff_lds(d) > 64 * 1024) {
     g_err = "scene too large for the adjoint's LDS budget";
     return bail(FT_ERR_INVALID_ARGUMENT);
@@ -2213,7 +2223,7 @@ int ft_diff_forward_device(ft_diff* d, void* t_dev, void* s_dev) {
   if (t_dev) FT_HIP(hipMemcpyAsync(t_dev, d->t.ptr, bytes, hipMemcpyDeviceToDevice, d->stream));
   if (s_dev) FT_HIP(hipMemcpyAsync(s_dev, d->s.ptr, bytes, hipMemcpyDeviceToDevice, d->stream));
   d->stats.primary_rays = diff_pixels(d);
-  d->stats.kernel_launches = 2;
+  d->stats.kernel_launches = d->n_prims > 1 ? 2 : 1;
   return FT_OK;
 }
 
@@ -2306,7 +2316,7 @@ int ft_diff_fit(ft_diff* d, uint32_t steps, float lr, float wt, float ws, double
   float ms = 0.0f;
   FT_HIP(hipEventElapsedTime(&ms, d->ev0, d->ev1));
   d->stats.last_kernel_ms = ms;
-  d->stats.kernel_launches = (uint64_t)steps * 8;
+  d->stats.kernel_launches = (uint64_t)steps * (d->n_prims > 1 ? 8 : 7);
   d->stats.primary_rays = (uint64_t)steps * diff_pixels(d);
   if (losses_out) FT_HIP(hipMemcpy(losses_out, d->losses.ptr, steps * sizeof(double), hipMemcpyDeviceToHost));
   return FT_OK;

@@ -38,6 +38,13 @@ constexpr unsigned long long kDiffAccSphere = 29, kDiffAccJoin = 10;
 //   x: sphere index, what follows it: kDiffJoin a join, kDiffPrim the sphere itself, the operand
 //      left over at the join (kOneShift), the join's index
 //   y: the join's radius max(|k|, 1e-6) as a float
+// kDiffCells by the time of a forward / of a gradient step in us, the building in it:
+//   cells   8 spheres 2x64^2   32 spheres 4x256^2   32 spheres 16x512^2   48 spheres 4x256^2
+//   24      400 / 700          1650 / 3070          4290 / 7590           2310 / 4730
+//   32      365 / 665          1370 / 2560          3700 / 6610           1990 / 4090
+//   48      350 / 615          1160 / 2190          3200 / 5630           1650 / 3350
+//   64      360 / 605          1090 / 2080          3100 / 5380           1580 / 3130
+// 64 takes 2.4 times the memory (199 MB at 48 spheres) and building time for the last few percent.
 constexpr int kDiffCells = 48;
 constexpr int kDiffStack = 8;       // values below the top: balanced trees of up to 48 spheres
 constexpr unsigned kDiffIndex = 0xffu, kDiffPrim = 1u << 31, kDiffJoin = 1u << 30;

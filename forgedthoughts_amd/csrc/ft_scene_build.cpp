@@ -186,13 +186,17 @@ void plan_grid(HostScene& S, double target) {
     S.cell_parents[k] = std::max(1, (int)std::ceil(ext[k] / (side * ftd::kCellChildrenSide)));
   }
   // a distance is a handful of f32 operations on coordinates of at most `scale`: a few ulp,
-  // covered ten times over
+  // covered ten times over.  Primitives that a hard boolean cuts with may lie far beyond the bounds;
+  // a cell's choice is then off by no more than their distances themselves are rounded.
   S.cell_margin = (float)(1.0e-5 * scale);
 }
 
-// The leaf lists of a multi-leaf scene in the accelerated modes: from 16 leaves on (below, a BVH
-// walk of the wave is a handful of nodes), where most leaves are primitives that the lists
-// evaluate themselves.  Finer cells keep shorter lists: of a 4097-leaf Whitted frame / a
+// The leaf lists of a multi-leaf scene in the accelerated modes: from 16 leaves on, where most
+// leaves are primitives that the lists evaluate themselves.  BVH walk against lists, preview at 96x96
+// and Whitted at 640x360 and 4 samples, ms: 16 leaves 0.99-1.7 / 0.27-0.38 and 2.0-2.6 / 0.88-0.99, 20
+// leaves 1.8-2.4 / 0.30-0.44 and 2.7-3.6 / 1.0-1.2, 300 in a clump 11.4 / 0.35 and 18.3 / 1.2, with a
+// fifth of them outside the common form 5.1 / 1.2 and 16.3 / 4.7.  9 to 14 leaves gain too (0.54-1.6 /
+// 0.23-0.38, 1.2-2.3 / 0.78-0.97): the line could be lower.  Finer cells keep shorter lists: of a 4097-leaf Whitted frame / a
 // 1501-leaf preview (27.1 / 1.87 ms at 8 cells a leaf) 32 took 20.1 / 1.25 ms, 128
 // 17.6 / 1.01 ms and 256 16.8 / 0.95 ms; past 128 the memory doubles for a few percent.
 constexpr size_t kMinListLeaves = 16;
@@ -230,7 +234,9 @@ void plan_leaf_lists(HostScene& S) {
 }
 
 // The cell programs of a scene that is one tree of the operators whose reach they know, from
-// 8 primitives on (the smallest scenes of the batch workload).  64^3 cells: 12 scenes of 8 to
+// 8 primitives on, where tiny words end.  Node program against cells, preview and Whitted at 640x360 (ms): 8
+// parts 0.80-1.25 / 0.20-0.35 and 1.3-1.9 / 0.37-0.46, closely packed 1.1-1.2 / 0.47-0.59 and 1.5-1.7 /
+// 0.75-0.86, 64 packed 9.0-9.3 / 1.8-2.7 and 12-14 / 2.4-4.0 (straight-line code: ft_backend.hip).  64^3 cells: 12 scenes of 8 to
 // 2048 primitives, four views each, took 39.0 ms a batch with 16 384 cells a scene, 24.5 with
 // 32 768, 17.3, 13.0 and 10.9 ms with 262 144 (about 30 MB a scene).
 constexpr int kMinCellNodes = 15;
