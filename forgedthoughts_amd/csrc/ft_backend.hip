@@ -1987,6 +1987,16 @@ void diff_bounds_host(const float* th, uint32_t n, uint32_t n_params, float out[
 
 constexpr size_t kDiffCellCount = (size_t)kDiffCells * kDiffCells * kDiffCells + 1;  // and the whole tree
 
+unsigned diff_waves(const ft_diff* d) {
+  return (unsigned)((size_t)d->n_views * ((((int)d->opts.width + 7) / 8) * (((int)d->opts.height + 7) / 8)));
+}
+// Tiles that a wave of the adjoint takes one after the other: one, so that small images keep the chip
+// busy, but for images whose partial sums (a row of doubles per wave) would take more than some 100 MB.
+// 1 / 2 / 4 tiles, us of a backward: 8 spheres 1x32^2 89-108 / 120-179 / 157-218, 40 spheres 1x128^2
+// 394-434 / 636-672 / 991-1054, 32 spheres 2x512^2 441-460 / 576-590 / 964, 16x512^2 1745-2086 /
+// 2115-2251 / 2251-2432.
+constexpr unsigned kDiffAdjointWaves = 65536;
+unsigned diff_wave_tiles(const ft_diff* d) { return std::max(1u, (diff_waves(d) + kDiffAdjointWaves - 1) / kDiffAdjointWaves); }
 DiffArgs diff_args(ft_diff* d) {
   DiffArgs a;
   a.nodes = (const int4*)d->nodes.ptr;
@@ -2000,6 +2010,7 @@ DiffArgs diff_args(ft_diff* d) {
   a.n_params = (int)d->n_params;
   a.n_views = (int)d->n_views;
   a.tiles_per_view = (((int)d->opts.width + 7) / 8) * (((int)d->opts.height + 7) / 8);
+  a.wave_tiles = (int)diff_wave_tiles(d);
   a.max_steps = (int)d->opts.max_steps;
   a.eps = d->opts.epsilon;
   a.step_scale = d->opts.step_scale;
@@ -2015,10 +2026,7 @@ DiffArgs diff_args(ft_diff* d) {
 size_t diff_lds(const ft_diff* d) {
   return ((size_t)2 * ((d->n_params + 1) & ~1u) + (size_t)(kDiffStack + 2 * kDiffKept) * 64) * sizeof(float);
 }
-unsigned diff_waves(const ft_diff* d) {
-  return (unsigned)((size_t)d->n_views * ((((int)d->opts.width + 7) / 8) * (((int)d->opts.height + 7) / 8)));
-}
-unsigned diff_blocks(const ft_diff* d) { return (diff_waves(d) + kDiffTiles - 1) / kDiffTiles; }  // of the adjoint
+unsigned diff_blocks(const ft_diff* d) { return (diff_waves(d) + diff_wave_tiles(d) - 1) / diff_wave_tiles(d); }  // of the adjoint
 size_t diff_pixels(const ft_diff* d) { return (size_t)d->n_views * d->opts.width * d->opts.height; }
 
 void diff_build_cells(ft_diff* d) {

@@ -61,6 +61,7 @@ struct DiffArgs {
   int max_steps;
   float eps, step_scale, max_dist, normal_step;
   float lx, ly, lz;       // unit light direction
+  int wave_tiles;         // of a wave of the adjoint
 };
 
 // Which product of a sum is fused is written out: left to the compiler it depends on the code
@@ -586,10 +587,9 @@ __device__ __forceinline__ bool interior_hit(const float* __restrict__ t, int w,
 }
 
 // Adjoint: accumulates sum over pixels of dL/dth into per-block partial sums (FP64): one wave
-// per block, kDiffTiles tiles one after the other, so a block's sums are added in a fixed order.
+// per block, wave_tiles tiles one after the other, so a block's sums are added in a fixed order.
 // kCounted adds the passes of the lanes with a non-zero upstream gradient to *flops.
 // LDS: gradient accumulator [n_params doubles], value stacks, kept operands.
-constexpr int kDiffTiles = 4;
 template <bool kCounted>
 __device__ __forceinline__ void diff_adjoint_body(DiffArgs a, const float* __restrict__ t_img,
                                                   const float* __restrict__ gt_img, const float* __restrict__ gs_img,
@@ -603,8 +603,8 @@ __device__ __forceinline__ void diff_adjoint_body(DiffArgs a, const float* __res
   DiffStart start;
   DiffTrace tr;
   tr.lds = stack + kDiffStack * 64 + lane;
-  for (int it = 0; it < kDiffTiles; ++it) {
-    const int w = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kDiffTiles + it);
+  for (int it = 0; it < a.wave_tiles; ++it) {
+    const int w = __builtin_amdgcn_readfirstlane((int)blockIdx.x * a.wave_tiles + it);
     const int view = w / a.tiles_per_view, tile = w - view * a.tiles_per_view;
     if (view >= a.n_views) break;
     const CamArgs cam = load_uniform(uniform_ptr(a.cams) + view);

@@ -262,3 +262,31 @@ def test_loss_is_that_of_the_whole_tree(seed):
         loss, _ = dr.loss_grad()
     want = WHOLE_TREE_LOSS[seed]
     assert abs(loss - want) <= 2.0 ** -20 * math.sqrt(4 * 320 * 320 * want), (loss, want)
+
+
+def test_adjoint_of_more_tiles_than_waves():
+    """Beyond 65536 tiles a wave of the adjoint takes several, the last ones of it none: the gradient is the
+    sum of those of its views' halves, to the order of the double sums."""
+    import torch
+    opts = RenderOptions(width=130, height=130, max_steps=64, max_dist=30.0, epsilon=1e-3, step_scale=0.7,
+                         camera_z=6.0, fov_y_degrees=45.0)
+    n = 230  # views of 17 x 17 tiles: 66470 in all
+    rng = np.random.default_rng(4)
+    params = np.float32([-0.4, 0.1, 0.0, 0.7, 0.5, -0.1, 0.2, 0.6, 0.2])
+    views = []
+    for k in range(n):
+        phi = 2 * np.pi * k / n
+        views.append((0, (5 * np.cos(phi), 1.0, 5 * np.sin(phi)), (0.0, 0.0, 0.0), 45.0))
+    up = np.float32(rng.normal(size=(2, n, 130, 130)))
+    print(f"[diff adjoint] {n} views at 130^2", flush=True)
+
+    def gradient(lo, hi):
+        with DiffRenderer(2, views[lo:hi], opts) as dr:
+            dr.set_params(params)
+            dr.forward()
+            gt, gs = (torch.from_numpy(np.ascontiguousarray(u[lo:hi])).cuda() for u in up)
+            torch.cuda.synchronize()
+            return dr.backward_device(gt.data_ptr(), gs.data_ptr())
+    whole, parts = gradient(0, n), gradient(0, n // 2) + gradient(n // 2, n)
+    assert np.abs(whole).max() > 1.0
+    np.testing.assert_allclose(whole, parts, rtol=1e-9, atol=1e-9 * np.abs(whole).max())
