@@ -474,7 +474,7 @@ int ft_scene_stats(ft_scene* scene, ft_render_stats* out);
  * caller of those entry points would otherwise issue as one call per (scene, view).
  * Every view of a call has the options' image size and the settings' sample count; its
  * camera replaces the scene's `camera` binding (parse_camera renderer.rs:6263-6286).
- * Scenes of a batch run on the node-program interpreter (no per-scene compilation). */
+ * Scenes of a batch are never compiled: they run on their cells, their node program or the BVH. */
 typedef struct ft_batch ft_batch;
 
 typedef struct ft_view {
