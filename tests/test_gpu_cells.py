@@ -280,14 +280,25 @@ def test_noalloc_with_cells_needs_a_built_kernel():
 def test_stats_say_when_kernels_are_built():
     """A tree with cells, no function, and an intersection of unlike materials: of its kernels only
     the shading sweep is compiled, and the flags have to say that one is."""
+    import ctypes
+    import torch
+    from forgedthoughts_amd.render import library
     text = tree_scene(60, 21, (1.0, 2.0, -6.5), ["union_round", "and"], ("Lambert", "Metal"), plain=True)
     opts = RenderOptions(width=32, height=24, **OPTS)
+    o, rs = opts.to_c(), RaySettings(1, 64, 1).to_c()
+    rgb = torch.zeros(32 * 24 * 3, dtype=torch.uint8, device="cuda")
     with GpuScene(compile_src(text), AccelMode.Bvh) as gs:
         gs.render_depth(opts, 1)
         assert gs.stats().compile_ms == 0.0
         assert gs.stats().flags == abi.STATS_EMITTED_SCENE
+
+        def call():  # refused while the kernel has to be built (or loaded from the code cache)
+            return library().ft_render_whitted_device_noalloc(gs.handle, ctypes.addressof(o), ctypes.addressof(rs),
+                                                              rgb.data_ptr(), None)
+        assert call() != 0
         gs.render_whitted(opts, RaySettings(1, 64, 1))
-        assert gs.stats().compile_ms > 0.0
+        assert call() == 0
+        gs.synchronize()
 
 
 # (text of the scene after the camera and lights, eye): one primitive; every primitive kind, rotated
@@ -422,6 +433,34 @@ def test_without_memory_for_cells(case, mb, monkeypatch):
         for gs in held:
             gs.close()
         assert taken < 8 << 22, taken  # the cells' headers alone would be 6 MB a scene
+
+
+@pytest.mark.parametrize("accel", [AccelMode.Bvh, AccelMode.Naive])
+@pytest.mark.parametrize("kind", ["unlike", "hooks"])
+def test_cells_beside_a_compiled_sweep(kind, accel, monkeypatch):
+    """Trees whose distance comes from cells and whose shading sweep is compiled, since the cells' shading
+    words do not serve: a hard boolean of unlike materials, a material with a per-hit hook."""
+    if kind == "unlike":
+        text = tree_scene(60, 22, (1.0, 2.0, -6.5), ["union_round", "and"], ("Lambert", "Metal"), plain=True)
+    else:
+        text = tree_scene(40, 22, (1.0, 2.0, -6.5), JOINS[:4], plain=True, extent=4.0)
+        head, rest = text.split("let m0 = ", 1)
+        text = (head + "material Hooked { model: Lambert; fn color(ctx) { return ctx.normal * 0.5 + vec3(0.5); } };\n"
+                "let m0 = Hooked {}" + rest[rest.index(";"):])
+    scene = compile_src(text)
+    opts = RenderOptions(width=64, height=48, **OPTS)
+    print(f"[cells and a compiled sweep] {kind}, accel {int(accel)}", flush=True)
+    counts = []
+    for emit in ("auto", "0"):
+        monkeypatch.setenv("FT_EMIT", emit)
+        with GpuScene(scene, accel) as gs:
+            assert gs.stats().cells == abi.CELLS_PROGRAMS
+            assert (gs.stats().flags & abi.STATS_EMITTED_SCENE) == (abi.STATS_EMITTED_SCENE if emit == "auto" else 0)
+            against_oracle(scene, accel, gs, opts, kind, depth=1)
+            gs.set_flop_counting(True)
+            gs.render_depth(opts, 1)
+            counts.append(gs.stats().sdf_flops)
+    assert counts[0] == counts[1] > 0  # a small launch counts the cells: so does the Whitted kernel
 
 
 # nodes of the tree for each word of a cell on the surface: 7 of the 63, 14 of the 95, 20 of the 127
